@@ -15,6 +15,8 @@ namespace fcfd {
 constexpr int MAXK = 64;
 constexpr int MAXR = 512;   // reactions
 constexpr int MAXTB = 16;   // enhanced third bodies per reaction
+constexpr int SPECIES_BLOCKS = 4;   // blocks the fluid kernels split the species into, one per wave
+constexpr int MAXCLS = 8;   // temperature classes of a block
 
 #define FCFD_FOR_EACH_NSP(X) X(53) X(11)
 
@@ -30,6 +32,15 @@ struct DevThermo {
     double alo[MAXK][7];
     double ahi[MAXK][7];
     double h298[MAXK];      // CKHMS(298.15) erg/g, for heat-release diagnostics
+    double rwt[MAXK];       // 1 / wt, correctly rounded (the divisor's reciprocal in quot())
+    // Coefficient sets by temperature class, for the fluid kernels' species blocks (block w: species
+    // w*M .. w*M + M - 1, M = ceil(kk / SPECIES_BLOCKS)).  The temperature axis is cut at the distinct mid
+    // temperatures of the block's species: class c holds the T above exactly c of them, and one
+    // coefficient set per species serves the whole class.  nclass = 0 where a block has more than
+    // MAXCLS - 1 distinct mid temperatures.
+    int nclass[SPECIES_BLOCKS];
+    double cut[SPECIES_BLOCKS][MAXCLS];      // the nclass - 1 distinct mid temperatures, ascending
+    double coef[SPECIES_BLOCKS][MAXCLS][MAXK / SPECIES_BLOCKS][6];
 };
 
 // Host-side mechanism read from the CHEMKIN-II link files.
@@ -59,7 +70,7 @@ int load_mech(const char *chem_bin, const char *tran_bin, Mech &m, std::string &
 int load_mech_text(const char *chem_inp, const char *therm_dat, Mech &m, std::string &err);
 // TRANLIB fits of a tran.bin link file for the species of m (mech_io.cpp).
 int load_tran_bin(const char *tran_bin, Mech &m, std::string &err);
-void thermo_h298(DevThermo &t);
+void thermo_derived(DevThermo &t);
 
 void set_error(const std::string &msg);
 

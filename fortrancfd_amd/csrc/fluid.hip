@@ -4,7 +4,7 @@
 // owns columns [b*S, (b+1)*S), S = ncell + 2*lv; its interior cell i (0-based) is column
 // b*S + lv + i, exactly the reference's b_obj(ib)%qf(:, ista-lv : iend+lv) column range.
 // Interface j (0..ncell) of block b -- the reference's Fplus(:, ista-1+j) -- is F[v*PF + b*(ncell+1)+j].
-#include "fcfd_device.hpp"
+#include "fluid_coop.hpp"
 #include "fluid.hpp"
 
 namespace fcfd {
@@ -14,190 +14,283 @@ namespace fcfd {
 // primitive vector (SRC/flux.f90:247-268, SRC/eos.f90:11-46).
 // ---------------------------------------------------------------------------------------------
 struct Side {
-    double rho, u, T, sy, p, a, E;
+    double rho, u, p, a, E;
 };
 
-// y[k * stride] holds the reconstructed Y_k (a register array with stride 1 or an LDS column).  Over
-// an LDS column the species loops unroll by four only: fully unrolled, the advection-flux kernel
-// needs more than 256 registers and spills to scratch.
-template <int NSP, int STRIDE = 1>
-__device__ __forceinline__ Side side_state(const DevThermo *__restrict__ m, double rho, double u,
-                                           double T, const double *y) {
-    Side s;
-    s.rho = rho; s.u = u; s.T = T;
-    // adjust_sum(Y) denominator (Y itself is renormalised lazily where QcL/R needs it).
-    double sy = 0.0, syw = 0.0;
-#pragma unroll (STRIDE == 1 ? NSP : 4)
-    for (int k = 0; k < NSP; ++k) {
-        sy = sy + fmax(y[k * STRIDE], 0.0);
-        syw = syw + y[k * STRIDE] / m->wt[k];          // CKYTX on the raw reconstructed Y
-    }
-    s.sy = sy;
-    // mole fractions, clipped and renormalised (SRC/flux.f90:250-253), formed on the fly in the
-    // mixture sums instead of being held in an array: each sum keeps its species order, and the
-    // per-species quotient is the same expression every time it is formed
-    double sx = 0.0;
-#pragma unroll (STRIDE == 1 ? NSP : 4)
-    for (int k = 0; k < NSP; ++k) sx = sx + fmax(y[k * STRIDE] / (syw * m->wt[k]), 0.0);
-    const TPow tp = tpow(T, m->ru);
-    double wtm = 0.0;
-    MixSums ms{0.0, 0.0, 0.0};
-#pragma unroll (STRIDE == 1 ? NSP : 4)
-    for (int k = 0; k < NSP; ++k) {
-        const double xk = fmax(y[k * STRIDE] / (syw * m->wt[k]), 0.0) / sx;
-        wtm = wtm + xk * m->wt[k];                                   // mix_w
-        const Nasa a = nasa(m, k, T);                                // mix_sums
-        ms.ubml = ms.ubml + xk * (h_mol(a, tp) - tp.rut);
-        const double c = cp_mol(a, tp);
-        ms.cpbml = ms.cpbml + xk * c;
-        ms.cvbml = ms.cvbml + xk * (c - m->ru);
-    }
-    s.p = (rho * 1.e-3) * m->ru * T / wtm * 0.1;                 // pressure(), CKPX
-    const double e = ms.ubml * 1.e-4 / wtm;                      // specific_energy()
-    s.E = rho * (e + 0.5 * (u * u));
-    const double cp = ms.cpbml * 1.e-4 / wtm, cv = ms.cvbml * 1.e-4 / wtm;
-    s.a = sqrt(cp / cv * s.p / rho);                             // sonic_speed()
-    return s;
-}
-
-// ---------------------------------------------------------------------------------------------
-// calc_flux_advection: TWO LANES PER INTERFACE.  Lanes 2j and 2j+1 of a wave share interface j
-// of the wave's range: lane parity s = 0 builds the left state, s = 1 the right state (each
-// reconstructs the stencil, keeps its side's values and runs qfToQc / pressure / sonic speed on
-// them); the two side records and, per species, the two mass fractions are exchanged between the
-// pair (side records by a lane shuffle, mass fractions through LDS), both lanes evaluate the same
-// Riemann branch, and the flux components
-// are written alternately by the two lanes.  Every output is the same expression of the same
-// operands as in a one-lane evaluation, so the rounding is unchanged.
-// ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ double pair_other(double v) { return __shfl_xor(v, 1, 64); }
+__device__ __forceinline__ double pair_other(double v) { return __shfl_xor(v, 32, 64); }
 
 __device__ __forceinline__ Side pair_other(const Side &me) {
     Side o;
-    o.rho = pair_other(me.rho); o.u = pair_other(me.u); o.T = pair_other(me.T);
-    o.sy = pair_other(me.sy); o.p = pair_other(me.p); o.a = pair_other(me.a); o.E = pair_other(me.E);
+    o.rho = pair_other(me.rho); o.u = pair_other(me.u);
+    o.p = pair_other(me.p); o.a = pair_other(me.a); o.E = pair_other(me.E);
     return o;
 }
 
-template <int NSP, int RK, bool SPH, int BS = 64, int WPE = 2>
-__global__ void __launch_bounds__(BS, WPE) k_flux(FluxArgs a) {
-    const long g2 = long(xcd_block()) * blockDim.x + threadIdx.x;
-    const long g = g2 >> 1;                               // interface (pairs never straddle a wave)
-    const int s = int(threadIdx.x & 1);                   // 0: left state, 1: right state
-    const int nif = a.ncell + 1;
-    if (g >= long(a.nblk) * nif) return;                  // both lanes of a pair leave together
+// ---------------------------------------------------------------------------------------------
+// calc_flux_advection: 32 interfaces per workgroup of four waves.  Lanes 0..31 of every wave build
+// the left states of the workgroup's interfaces, lanes 32..63 the right states (the right-state
+// formulas are the left-state ones on the mirrored stencil); wave w reconstructs the species
+// w*M .. w*M + M - 1 and one of rho, u, T, and keeps its species in registers.  The mixture sums
+// run over the waves in species order (chain_sum); wave 0 completes the two side records, exchanges
+// them between the lane halves, evaluates the Riemann branch and the first three components, and
+// publishes what the species components need; with HLLC only the upwind side's lanes write those.
+// Every output is the same expression of the same operands as in a one-lane evaluation.
+//
+// Bound: FP64 issue (WENO weights, NASA-7 sums).  A whole side per lane, with its 53 mass fractions in
+// 27 KB of LDS per wave, left one wave per SIMD, full divisions and per-lane coefficient selects: 54 us
+// for 400 cells, 144 us for 65,536, 560 us for 262,144 (GRI-3.0, WENO5-JS + HLLC).  Split over four
+// waves (142 registers, three waves per SIMD), with scalar coefficients and quotients by shared
+// reciprocals: 16, 55 and 195 us.  The mass fractions wait in LDS while the sums run: kept in
+// registers they cost the third wave (236 us).
+// ---------------------------------------------------------------------------------------------
+template <int NSP, int RK, bool SPH, int RS, int WPE = 3>
+__global__ void __launch_bounds__(64 * GW, WPE) k_flux(FluxArgs a) {
+    constexpr int M = group_m<NSP>();
+    __shared__ CoopShared sh;
+    __shared__ double prim[3][64];                        // rho, u, T of this lane's side
+    __shared__ double pub[3][64];                         // the Riemann solution, for the species components
+    __shared__ double park[M][64 * GW];                   // each lane's mass fractions while the sums run
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int s = lane >> 5;                              // 0: left state, 1: right state
+    const unsigned nif = unsigned(a.ncell) + 1u, total = unsigned(a.nblk) * nif;
+    const unsigned g0 = xcd_block() * 32u + unsigned(lane & 31);
+    const bool live = g0 < total;
+    const unsigned g = live ? g0 : total - 1u;            // lanes past the end shadow the last interface
     // a launch covers blocks b0 .. b0 + nblk - 1 (the coarse blocks of a refined mesh reconstruct
     // at first order in launches of their own, SRC/flux.f90:240)
-    const int b = a.b0 + int(g / nif), j = int(g % nif);
-    const long gi = long(b) * nif + j;                    // interface index over all blocks
-    const long c0 = long(b) * a.S + a.lv + j - 1;      // left cell of the interface
-    const DevThermo *__restrict__ m = a.thermo;
+    const unsigned bl = g / nif, j0 = g - bl * nif;
+    const unsigned gi = (unsigned(a.b0) + bl) * nif + j0; // interface index over all blocks
+    const unsigned c0 = (unsigned(a.b0) + bl) * unsigned(a.S) + unsigned(a.lv) + j0 - 1u;   // its left cell
+    CThermo *m = constant(a.thermo);
     const double *__restrict__ q = a.qf;
 
-    // each lane reconstructs its own side only
-    const double rho_s = reconstruct_side<RK>(q + 0 * a.P, c0, a.muscl, s);
-    const double u_s = reconstruct_side<RK>(q + 1 * a.P, c0, a.muscl, s);
-    const double T_s = reconstruct_side<RK>(q + 2 * a.P, c0, a.muscl, s);
-    // reconstructed mass fractions of this lane's side, species-major in LDS (column = lane)
-    __shared__ double ys[NSP * BS];
-    double *y = ys + threadIdx.x;
-    for (int k = 0; k < NSP; ++k) y[k * BS] = reconstruct_side<RK>(q + (3 + k) * a.P, c0, a.muscl, s);
-    const double *yo_col = ys + (threadIdx.x ^ 1);     // the pair partner's side
-    const Side me = side_state<NSP, BS>(m, rho_s, u_s, T_s, y);
-    const Side ot = pair_other(me);
-    const Side L = s ? ot : me;
-    const Side R = s ? me : ot;
+    double y[M];
+    if constexpr (RK == R_WENO5JS || RK == R_WENO5Z) {
+        // byte offsets of the side's stencil: left q[c0 - 2 .. c0 + 2], right q[c0 + 3 .. c0 - 1]
+        unsigned o[5];
+#pragma unroll
+        for (int i = 0; i < 5; ++i) o[i] = (c0 + unsigned(s ? 3 - i : i - 2)) * 8u;
+        bool big = false;
+        // two variables' stencils in flight ahead of the one being reconstructed (more would spill)
+        auto row = [&](int j) { return q + long(j < 0 ? min(w, 2) : 3 + min(w * M + j, NSP - 1)) * a.P; };
+        double v[2][5];
+        load5(row(-1), o, v[0]);
+        load5(row(0), o, v[1]);
+#pragma unroll
+        for (int j = -1; j < M; ++j) {
+            double r = weno5_lane<RK>(v[(j + 1) & 1], s, big);
+            asm volatile("" : "+v"(r));                   // finished here, not behind the test of big
+            if (j < 0) { if (w < 3) prim[w][lane] = r; }
+            else y[j] = r;
+            if (j + 2 < M) load5(row(j + 2), o, v[(j + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (__any(big)) {                                 // far out of any gas: with plain divisions
+            if (w < 3) prim[w][lane] = reconstruct_side<RK>(q + long(w) * a.P, c0, a.muscl, s);
+#pragma unroll
+            for (int j = 0; j < M; ++j) {
+                y[j] = reconstruct_side<RK>(q + long(3 + min(w * M + j, NSP - 1)) * a.P, c0, a.muscl, s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    } else {
+        if (w < 3) prim[w][lane] = reconstruct_side<RK>(q + long(w) * a.P, c0, a.muscl, s);
+#pragma unroll
+        for (int j = 0; j < M; ++j) y[j] = reconstruct_side<RK>(q + long(3 + min(w * M + j, NSP - 1)) * a.P, c0, a.muscl, s);
+    }
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        y[j] = w * M + j < NSP ? y[j] : 0.0;
+        ok = ok && num_ok(y[j]);
+    }
+    const bool fast = __all(ok);
+    double sy, syw;
+    {
+        double yw[M], r[2];
+        over_wt_coop<NSP>(m, w, fast, y, yw);             // CKYTX on the raw reconstructed Y
+        // (its barriers also publish prim)
+        chain_sum<2, M>(sh.c[0], w, lane, [&](int c, int j) { return c == 0 ? fmax(y[j], 0.0) : yw[j]; }, r);
+        sy = r[0];                                        // adjust_sum(Y) denominator
+        syw = r[1];
+    }
+    const double rho = prim[0][lane], u = prim[1][lane], T = prim[2][lane];
+    double mix[4];                                        // mean molar mass, u, cp, cv (molar)
+    {
+        // mole fractions, clipped and renormalised (SRC/flux.f90:250-253)
+        double x[M], r[1];
+        ytx_coop<NSP>(m, w, fast, syw, y, x);
+#pragma unroll
+        for (int j = 0; j < M; ++j) park[j][threadIdx.x] = y[j];
+#pragma unroll
+        for (int j = 0; j < M; ++j) x[j] = fmax(x[j], 0.0);
+        chain_sum<1, M>(sh.c[1], w, lane, [&](int, int j) { return x[j]; }, r);
+        scale_coop<M>(fast, r[0], x);
+        double hu[M], cp[M];
+        species_thermo<NSP, true, true>(m, w, T, __all(den_ok(T)), hu, cp);
+        const double ru = m->ru;
+        // the products are formed as they are added: the terms of four sums would not fit beside y
+        chain_sum<4, M>(sh.c[0], w, lane, [&](int c, int j) {
+            return x[j] * (c == 0 ? m->wt[min(w * M + j, NSP - 1)] : c == 1 ? hu[j] : c == 2 ? cp[j] : cp[j] - ru);
+        }, mix);
+    }
 
-    // physical fluxes of mass, momentum, energy (SRC/flux.f90:270-280)
-    const double fl0 = L.rho * L.u, fr0 = R.rho * R.u;
-    // spherical: no pressure in the momentum flux; the update adds its gradient (SRC/flux.f90:272-278)
-    const double fl1 = SPH ? L.rho * L.u * L.u : L.rho * L.u * L.u + L.p;
-    const double fr1 = SPH ? R.rho * R.u * R.u : R.rho * R.u * R.u + R.p;
-    const double fl2 = (L.E + L.p) * L.u, fr2 = (R.E + R.p) * R.u;
-    double *__restrict__ F = a.F + gi;
+    double *__restrict__ F = a.F;
     const long PF = a.PF;
     // Fplus accumulates (SRC/flux.f90:358): on top of the transport flux when there is one
     const bool acc = a.accumulate != 0;
-    // component v is written by lane parity v & 1
-    auto put = [acc, s](double &d, int v, double val) {
-        if ((v & 1) == s) d = acc ? d + val : val;
+    auto put = [acc](double *row, unsigned at, double val) {
+        double *d = reinterpret_cast<double *>(reinterpret_cast<char *>(row) + at);
+        *d = acc ? *d + val : val;
     };
-
-    if (a.riemann == 0) {                                         // LxF (SRC/flux.f90:291-294)
-        const double lL = fmax(fmax(fabs(L.u - L.a), fabs(L.u)), fabs(L.u + L.a));
-        const double lR = fmax(fmax(fabs(R.u - R.a), fabs(R.u)), fabs(R.u + R.a));
-        const double al = fmax(lL, lR);
-        put(F[0], 0, 0.5 * (fl0 + fr0 - al * (R.rho - L.rho)));
-        put(F[PF], 1, 0.5 * (fl1 + fr1 - al * (R.rho * R.u - L.rho * L.u)));
-        put(F[2 * PF], 2, 0.5 * (fl2 + fr2 - al * (R.E - L.E)));
-#pragma unroll 4
-        for (int k = 0; k < NSP; ++k) {
-            const double ym = y[k * BS], yo = yo_col[k * BS];
-            const double yl = s ? yo : ym, yr = s ? ym : yo;
-            const double QL = L.rho * (fmax(yl, 0.0) / L.sy), QR = R.rho * (fmax(yr, 0.0) / R.sy);
-            const double fL = L.rho * yl * L.u, fR = R.rho * yr * R.u;
-            put(F[(3 + k) * PF], 3 + k, 0.5 * (fL + fR - al * (QR - QL)));
-        }
-    } else {
-        const double rt = sqrt(R.rho / L.rho);
-        const double uro = (L.u + rt * R.u) / (1.0 + rt);
-        const double aro = (L.a + rt * R.a) / (1.0 + rt);
-        const double sL = fmin(L.u - L.a, uro - aro), sR = fmax(R.u + R.a, uro + aro);
-        if (a.riemann == 1) {                                     // HLL (SRC/flux.f90:300-315)
-            int br = (0.0 <= sL) ? 0 : ((sL <= 0.0 && 0.0 <= sR) ? 1 : 2);
-            auto hll = [&](double fL, double fR, double QL, double QR) {
-                return br == 0 ? fL : (br == 1 ? (sR * fL - sL * fR + sL * sR * (QR - QL)) / (sR - sL) : fR);
-            };
-            put(F[0], 0, hll(fl0, fr0, L.rho, R.rho));
-            put(F[PF], 1, hll(fl1, fr1, L.rho * L.u, R.rho * R.u));
-            put(F[2 * PF], 2, hll(fl2, fr2, L.E, R.E));
-#pragma unroll 4
-            for (int k = 0; k < NSP; ++k) {
-                const double ym = y[k * BS], yo = yo_col[k * BS];
-                const double yl = s ? yo : ym, yr = s ? ym : yo;
-                const double QL = L.rho * (fmax(yl, 0.0) / L.sy), QR = R.rho * (fmax(yr, 0.0) / R.sy);
-                put(F[(3 + k) * PF], 3 + k, hll(L.rho * yl * L.u, R.rho * yr * R.u, QL, QR));
+    const unsigned gb = gi * 8u;
+    if (w == 0) {
+        Side me;
+        me.rho = rho; me.u = u;
+        const double wtm = mix[0];
+        me.p = (rho * 1.e-3) * m->ru * T / wtm * 0.1;                // pressure(), CKPX
+        const double e = mix[1] * 1.e-4 / wtm;                       // specific_energy()
+        me.E = rho * (e + 0.5 * (u * u));
+        const double cp = mix[2] * 1.e-4 / wtm, cv = mix[3] * 1.e-4 / wtm;
+        me.a = sqrt(cp / cv * me.p / rho);                           // sonic_speed()
+        const Side ot = pair_other(me);
+        const Side L = s ? ot : me;
+        const Side R = s ? me : ot;
+        // physical fluxes of mass, momentum, energy (SRC/flux.f90:270-280)
+        const double fl0 = L.rho * L.u, fr0 = R.rho * R.u;
+        // spherical: no pressure in the momentum flux; the update adds its gradient (SRC/flux.f90:272-278)
+        const double fl1 = SPH ? L.rho * L.u * L.u : L.rho * L.u * L.u + L.p;
+        const double fr1 = SPH ? R.rho * R.u * R.u : R.rho * R.u * R.u + R.p;
+        const double fl2 = (L.E + L.p) * L.u, fr2 = (R.E + R.p) * R.u;
+        double f0, f1, f2;
+        if (RS == 0) {                                                // LxF (SRC/flux.f90:291-294)
+            const double lL = fmax(fmax(fabs(L.u - L.a), fabs(L.u)), fabs(L.u + L.a));
+            const double lR = fmax(fmax(fabs(R.u - R.a), fabs(R.u)), fabs(R.u + R.a));
+            const double al = fmax(lL, lR);
+            f0 = 0.5 * (fl0 + fr0 - al * (R.rho - L.rho));
+            f1 = 0.5 * (fl1 + fr1 - al * (R.rho * R.u - L.rho * L.u));
+            f2 = 0.5 * (fl2 + fr2 - al * (R.E - L.E));
+            pub[0][lane] = al;
+        } else {
+            const double rt = sqrt(R.rho / L.rho);
+            const double uro = (L.u + rt * R.u) / (1.0 + rt);
+            const double aro = (L.a + rt * R.a) / (1.0 + rt);
+            const double sL = fmin(L.u - L.a, uro - aro), sR = fmax(R.u + R.a, uro + aro);
+            if (RS == 1) {                                            // HLL (SRC/flux.f90:300-315)
+                const int br = (0.0 <= sL) ? 0 : ((sL <= 0.0 && 0.0 <= sR) ? 1 : 2);
+                auto hll = [&](double fL, double fR, double QL, double QR) {
+                    return br == 0 ? fL : (br == 1 ? (sR * fL - sL * fR + sL * sR * (QR - QL)) / (sR - sL) : fR);
+                };
+                f0 = hll(fl0, fr0, L.rho, R.rho);
+                f1 = hll(fl1, fr1, L.rho * L.u, R.rho * R.u);
+                f2 = hll(fl2, fr2, L.E, R.E);
+                pub[0][lane] = sL;
+                pub[1][lane] = sR;
+                pub[2][lane] = double(br);
+            } else {                                                  // HLLC (SRC/flux.f90:321-354)
+                const double sM = (L.p - R.p + R.rho * R.u * (sR - R.u) - L.rho * L.u * (sL - L.u)) /
+                                  (R.rho * (sR - R.u) - L.rho * (sL - L.u));
+                // branch chain of SRC/flux.f90:332-354
+                const int br = (0.0 <= sL) ? 0 : ((sL <= 0.0 && 0.0 <= sM) ? 1 : ((sM <= 0.0 && 0.0 <= sR) ? 2 : 3));
+                const bool left = br <= 1;
+                const Side S = left ? L : R;
+                f0 = left ? fl0 : fr0;
+                f1 = left ? fl1 : fr1;
+                f2 = left ? fl2 : fr2;
+                // 0: this lane's side is not the upwind one; 1: supersonic, upwind flux; 2: star state
+                double mode = left == (s == 0) ? 1.0 : 0.0;
+                if (!(br == 0 || br == 3)) {                          // star state of the upwind side
+                    const double sK = left ? sL : sR;
+                    const double c = S.rho * (sK - S.u) / (sK - sM);
+                    const double v2 = S.E / S.rho + (sM - S.u) * (sM + S.p / (S.rho * (sK - S.u)));
+                    f0 = f0 + sK * (c * 1.0 - S.rho);
+                    f1 = f1 + sK * (c * sM - S.rho * S.u);
+                    f2 = f2 + sK * (c * v2 - S.E);
+                    mode = 2.0 * mode;
+                    pub[1][lane] = sK;
+                    pub[2][lane] = c;
+                }
+                pub[0][lane] = live ? mode : 0.0;
             }
-        } else {                                                  // HLLC (SRC/flux.f90:321-354)
-            const double sM = (L.p - R.p + R.rho * R.u * (sR - R.u) - L.rho * L.u * (sL - L.u)) /
-                              (R.rho * (sR - R.u) - L.rho * (sL - L.u));
-            // branch chain of SRC/flux.f90:332-354
-            const int br = (0.0 <= sL) ? 0 : ((sL <= 0.0 && 0.0 <= sM) ? 1 : ((sM <= 0.0 && 0.0 <= sR) ? 2 : 3));
-            const bool left = br <= 1;
-            const Side S = left ? L : R;
-            const double f0 = left ? fl0 : fr0, f1 = left ? fl1 : fr1, f2 = left ? fl2 : fr2;
-            if (br == 0 || br == 3) {                             // supersonic: upwind flux
-                put(F[0], 0, f0);
-                put(F[PF], 1, f1);
-                put(F[2 * PF], 2, f2);
-#pragma unroll 4
-                for (int k = 0; k < NSP; ++k) {
-                    const double yk = (left == (s == 0)) ? y[k * BS] : yo_col[k * BS];
-                    put(F[(3 + k) * PF], 3 + k, S.rho * yk * S.u);
-                }
-            } else {                                              // star state of the upwind side
-                const double sK = left ? sL : sR;
-                const double c = S.rho * (sK - S.u) / (sK - sM);
-                const double v2 = S.E / S.rho + (sM - S.u) * (sM + S.p / (S.rho * (sK - S.u)));
-                put(F[0], 0, f0 + sK * (c * 1.0 - S.rho));
-                put(F[PF], 1, f1 + sK * (c * sM - S.rho * S.u));
-                put(F[2 * PF], 2, f2 + sK * (c * v2 - S.E));
-#pragma unroll 4
-                for (int k = 0; k < NSP; ++k) {
-                    const double yk = (left == (s == 0)) ? y[k * BS] : yo_col[k * BS];
-                    const double Qk = S.rho * (fmax(yk, 0.0) / S.sy);
-                    const double fk = S.rho * yk * S.u;
-                    put(F[(3 + k) * PF], 3 + k, fk + sK * (c * (Qk / S.rho) - Qk));
-                }
+        }
+        if (live) {
+            if (s == 0) {
+                put(F, gb, f0);
+                put(F + 2 * PF, gb, f2);
+            } else {
+                put(F + PF, gb, f1);
+            }
+            if (a.godunov && s == 0) {                                // SRC/flux.f90:360-367
+                const double rt = sqrt(R.rho / L.rho);
+                double *G = a.godunov + gi;
+                G[0] = sqrt(R.rho * L.rho);
+                G[PF] = (L.u + rt * R.u) / (1.0 + rt);
+                G[2 * PF] = (L.p + rt * R.p) / (1.0 + rt);
             }
         }
     }
-    if (a.godunov && s == 0) {                                    // SRC/flux.f90:360-367
-        const double rt = sqrt(R.rho / L.rho);
-        double *G = a.godunov + gi;
-        G[0] = sqrt(R.rho * L.rho);
-        G[PF] = (L.u + rt * R.u) / (1.0 + rt);
-        G[2 * PF] = (L.p + rt * R.p) / (1.0 + rt);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < M; ++j) y[j] = park[j][threadIdx.x];
+    // adjust_sum(Y) where QcL/R needs it: Q_k = rho (max(Y_k, 0) / sy)
+    const bool fd = fast && __all(den_ok(sy) && den_ok(rho));
+    const double rsy = recip(sy), rrho = recip(rho);
+    if (RS == 2) {
+        const double mode = pub[0][lane], sK = pub[1][lane], c = pub[2][lane];
+        // star state: F + s_K (c Q_k / rho - Q_k); supersonic: the upwind flux
+        double f[M];
+        if (__any(mode == 2.0)) {
+            if (fd) {
+#pragma unroll
+                for (int j = 0; j < M; ++j) {
+                    const double Qk = rho * quot(fmax(y[j], 0.0), sy, rsy);
+                    f[j] = rho * y[j] * u + sK * (c * quot(Qk, rho, rrho) - Qk);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < M; ++j) {
+                    const double Qk = rho * (fmax(y[j], 0.0) / sy);
+                    f[j] = rho * y[j] * u + sK * (c * (Qk / rho) - Qk);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        if (__any(mode == 1.0)) {
+#pragma unroll
+            for (int j = 0; j < M; ++j) f[j] = mode == 1.0 ? rho * y[j] * u : f[j];
+        }
+        if (mode != 0.0) {
+            if (acc) {
+#pragma unroll
+                for (int j = 0; j < M; ++j)
+                    if (w * M + j < NSP) f[j] = at_byte(F + long(3 + w * M + j) * PF, gb) + f[j];
+            }
+#pragma unroll
+            for (int j = 0; j < M; ++j)
+                if (w * M + j < NSP) *reinterpret_cast<double *>(reinterpret_cast<char *>(F + long(3 + w * M + j) * PF) + gb) = f[j];
+        }
+    } else {
+        // both sides enter: this lane's Q_k and physical flux go to the interface's other lane, and
+        // the two lanes write alternate species
+        const double w0 = pub[0][lane], w1 = pub[1][lane], w2 = pub[2][lane];
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const int k = w * M + j;
+            if (k >= NSP) break;
+            const double yc = fmax(y[j], 0.0);
+            const double Qm = rho * (fd ? quot(yc, sy, rsy) : yc / sy), fm = rho * y[j] * u;
+            const double Qo = pair_other(Qm), fo = pair_other(fm);
+            const double QL = s ? Qo : Qm, QR = s ? Qm : Qo, fL = s ? fo : fm, fR = s ? fm : fo;
+            if ((k & 1) != s || !live) continue;
+            double v;
+            if (RS == 0) {
+                v = 0.5 * (fL + fR - w0 * (QR - QL));
+            } else {
+                v = w2 == 0.0 ? fL : (w2 == 1.0 ? (w1 * fL - w0 * fR + w0 * w1 * (QR - QL)) / (w1 - w0) : fR);
+            }
+            put(F + (3 + k) * PF, gb, v);
+        }
     }
 }
 
@@ -241,24 +334,35 @@ __device__ __forceinline__ void ghost_source(const StageArgs &a, int b, int i, i
 // of SRC/timeintegration.f90:150-175 (or :48-56 for Euler), then update_boundary /
 // interpolation_block / QcToqf on every column (:201-215).  mode 0: Q = Qin - dt/dx*dF;
 // mode 1: Q = h1*Q0 + h2*(Qin - dt/dx*dF); mode 2: no update (ghost fill + QcToqf only).
-template <int NSP, int BS = 64, int WPE = 2>
-__global__ void __launch_bounds__(BS, WPE) k_stage_end(StageArgs a) {
-    const long c = long(xcd_block()) * blockDim.x + threadIdx.x;
-    if (c >= long(a.nblk) * a.S) return;
-    const int b = int(c / a.S), i = int(c % a.S) - a.lv;
+// 64 columns per workgroup of four waves, wave w with the species w*M .. w*M + M - 1.  Bound: the FP64
+// issue of the temperature Newton iteration and its chain from one iteration to the next.  One
+// lane per column (56 values in registers, the coefficients selected per lane) took 75 us however
+// few columns there were, 111 us for 65,536 and 382 us for 262,144; split over four waves (three per
+// SIMD) 29, 50 and 160 us.
+template <int NSP, int MODE, bool SPH, int WPE = 3>
+__global__ void __launch_bounds__(64 * GW, WPE) k_stage_end(StageArgs a) {
+    constexpr int M = group_m<NSP>();
+    __shared__ CoopShared sh;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const unsigned ncol = unsigned(a.nblk) * unsigned(a.S);
+    const unsigned cq = xcd_block() * 64u + unsigned(lane);
+    const unsigned c = min(cq, ncol - 1u);                // lanes past the end shadow the last column
+    const int b = int(c / unsigned(a.S)), i = int(c - unsigned(b) * unsigned(a.S)) - a.lv;
     const bool ghost = (i < 0 || i >= a.ncell);
-    if (a.ghosts_only && !ghost) return;
+    const bool live = cq < ncol && (ghost || !a.ghosts_only);
+    if (!__any(live)) return;                             // the same in the four waves
     int sb, si;
     double sgn;
     ghost_source(a, b, i, sb, si, sgn);
-    const long sc = long(sb) * a.S + a.lv + si;
-    const long fj = long(sb) * (a.ncell + 1) + si;
+    const unsigned sc = (unsigned(sb) * unsigned(a.S) + unsigned(a.lv + si)) * 8u;      // byte offsets
+    const unsigned fj = (unsigned(sb) * unsigned(a.ncell + 1) + unsigned(si)) * 8u;
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
     const double dx = a.dxb ? a.dxb[sb] : a.dx;         // the source cell's block spacing
     const double dtdx = dt / dx;
     // spherical (SRC/timeintegration.f90:58-72, 177-196): face areas (r -+ dx/2)^2 and volume
     // r^2 dx at the source cell's centre
-    const bool sph = a.spherical && a.mode != 2;
+    constexpr bool sph = SPH && MODE != 2;
     double Al = 0.0, Ar = 0.0, dtdV = 0.0;
     if (sph) {
         const double rm = a.xm[long(sb) * a.ncell + si];
@@ -267,25 +371,50 @@ __global__ void __launch_bounds__(BS, WPE) k_stage_end(StageArgs a) {
         Ar = tr * tr;
         dtdV = dt / (rm * rm * dx);
     }
-    double Qv[NSP + 3];
-#pragma unroll
-    for (int v = 0; v < NSP + 3; ++v) {
-        double Q;
-        if (a.mode == 2) {
-            Q = a.Qin[v * a.P + sc];
-        } else {
-            const double fr = a.F[v * a.PF + fj + 1], fl = a.F[v * a.PF + fj];
-            const double qi = a.Qin[v * a.P + sc];
+    auto value = [&](int v) {
+        const double qi = at_byte(a.Qin + long(v) * a.P, sc);
+        double Q = qi;
+        if (MODE != 2) {
+            const double *f = a.F + long(v) * a.PF;
+            const double fr = at_byte(f + 1, fj), fl = at_byte(f, fj);
             const double base = sph ? qi - dtdV * (Ar * fr - Al * fl) : qi - dtdx * (fr - fl);
-            if (a.mode == 0) Q = base;
-            else Q = a.h1 * a.Q0[v * a.P + sc] + a.h2 * base;
-            if (sph && v == 1) Q = Q - dtdx * (a.god[2 * a.PF + fj + 1] - a.god[2 * a.PF + fj]);
+            if (MODE == 0) Q = base;
+            else Q = a.h1 * at_byte(a.Q0 + long(v) * a.P, sc) + a.h2 * base;
         }
-        if (v == 1) Q = sgn < 0.0 ? -Q : Q;
-        Qv[v] = Q;
-        a.Qout[v * a.P + c] = Q;
+        return Q;
+    };
+    const double rho = value(0), rE = value(2);
+    double ru = value(1);
+    if (sph) ru = ru - dtdx * (at_byte(a.god + 2 * a.PF + 1, fj) - at_byte(a.god + 2 * a.PF, fj));
+    ru = sgn < 0.0 ? -ru : ru;
+    double q[M], u, T;
+    // (species past the last one: the last one's column, then 0, so that no load waits on a branch)
+#pragma unroll
+    for (int j = 0; j < M; ++j) q[j] = value(3 + min(w * M + j, NSP - 1));
+#pragma unroll
+    for (int j = 0; j < M; ++j) q[j] = w * M + j < NSP ? q[j] : 0.0;
+    const unsigned cb = c * 8u;
+    auto put = [cb, live](double *row, double v) {
+        if (live) *reinterpret_cast<double *>(reinterpret_cast<char *>(row) + cb) = v;
+    };
+    // a refresh runs in place (Qout = Qin): ghost columns read interior columns, whose owners write
+    // back the value they read
+    if (w == 0) {
+        put(a.Qout, rho);
+        put(a.Qout + a.P, ru);
+        put(a.Qout + 2 * a.P, rE);
     }
-    qc_to_qf_store<NSP>(a.thermo, Qv, a.qf, a.P, c);
+#pragma unroll
+    for (int j = 0; j < M; ++j)
+        if (w * M + j < NSP) put(a.Qout + long(3 + w * M + j) * a.P, q[j]);
+    qc_to_qf_coop<NSP>(constant(a.thermo), sh, w, lane, rho, ru, rE, q, u, T, [&](int j, double y) {
+        if (w * M + j < NSP) put(a.qf + long(3 + w * M + j) * a.P, y);
+    });
+    if (w == 0) {
+        put(a.qf, rho);
+        put(a.qf + a.P, u);
+        put(a.qf + 2 * a.P, T);
+    }
 }
 
 // RK4 stage (SRC/timeintegration.f90:222-356) with the reference's semantics: within the step the
@@ -564,29 +693,33 @@ static int recon_kind(int flag_acu, int flag_weno) {
     }
 }
 
-template <int NSP, bool SPH>
-static hipError_t launch_flux_nsp(const FluxArgs &a, int rk, hipStream_t st) {
-    const long n = 2 * long(a.nblk) * (a.ncell + 1);            // two lanes per interface
-    const dim3 grid(unsigned((n + 63) / 64)), blk(64);
-    const dim3 grid2(unsigned((n + 127) / 128)), blk2(128);
-    switch (rk) {
-        case R_FIRST: hipLaunchKernelGGL((k_flux<NSP, R_FIRST, SPH>), grid, blk, 0, st, a); break;
-        case R_MUSCL: hipLaunchKernelGGL((k_flux<NSP, R_MUSCL, SPH>), grid, blk, 0, st, a); break;
-        case R_WENO3Z: hipLaunchKernelGGL((k_flux<NSP, R_WENO3Z, SPH>), grid, blk, 0, st, a); break;
-        case R_WENO5JS:
-            if (a.variant == 1) hipLaunchKernelGGL((k_flux<NSP, R_WENO5JS, SPH, 64, 1>), grid, blk, 0, st, a);
-            else if (a.variant == 2) hipLaunchKernelGGL((k_flux<NSP, R_WENO5JS, SPH, 128, 1>), grid2, blk2, 0, st, a);
-            else hipLaunchKernelGGL((k_flux<NSP, R_WENO5JS, SPH>), grid, blk, 0, st, a);
+template <int NSP, bool SPH, int RK>
+static hipError_t launch_flux_rk(const FluxArgs &a, hipStream_t st) {
+    const long n = long(a.nblk) * (a.ncell + 1);
+    const dim3 grid(unsigned((n + 31) / 32)), blk(64 * GW);     // 32 interfaces, both sides, per workgroup
+    switch (a.riemann) {
+        case 0: hipLaunchKernelGGL((k_flux<NSP, RK, SPH, 0>), grid, blk, 0, st, a); break;
+        case 1: hipLaunchKernelGGL((k_flux<NSP, RK, SPH, 1>), grid, blk, 0, st, a); break;
+        default:
+            if constexpr (RK == R_WENO5JS || RK == R_WENO5Z)
+                if (a.variant == 1) { hipLaunchKernelGGL((k_flux<NSP, RK, SPH, 2, 4>), grid, blk, 0, st, a); break; }
+            hipLaunchKernelGGL((k_flux<NSP, RK, SPH, 2>), grid, blk, 0, st, a);
             break;
-        case R_WENO5Z:
-            if (a.variant == 1) hipLaunchKernelGGL((k_flux<NSP, R_WENO5Z, SPH, 64, 1>), grid, blk, 0, st, a);
-            else if (a.variant == 2) hipLaunchKernelGGL((k_flux<NSP, R_WENO5Z, SPH, 128, 1>), grid2, blk2, 0, st, a);
-            else hipLaunchKernelGGL((k_flux<NSP, R_WENO5Z, SPH>), grid, blk, 0, st, a);
-            break;
-        case R_WENO7Z: hipLaunchKernelGGL((k_flux<NSP, R_WENO7Z, SPH>), grid, blk, 0, st, a); break;
-        default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+template <int NSP, bool SPH>
+static hipError_t launch_flux_nsp(const FluxArgs &a, int rk, hipStream_t st) {
+    switch (rk) {
+        case R_FIRST: return launch_flux_rk<NSP, SPH, R_FIRST>(a, st);
+        case R_MUSCL: return launch_flux_rk<NSP, SPH, R_MUSCL>(a, st);
+        case R_WENO3Z: return launch_flux_rk<NSP, SPH, R_WENO3Z>(a, st);
+        case R_WENO5JS: return launch_flux_rk<NSP, SPH, R_WENO5JS>(a, st);
+        case R_WENO5Z: return launch_flux_rk<NSP, SPH, R_WENO5Z>(a, st);
+        case R_WENO7Z: return launch_flux_rk<NSP, SPH, R_WENO7Z>(a, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_smr_halo(const SmrArgs &a, int nsp, hipStream_t st) {
@@ -610,18 +743,20 @@ hipError_t launch_flux(const FluxArgs &a, int nsp, int flag_acu, int flag_weno, 
     return hipErrorInvalidValue;
 }
 
+template <int NSP, int MODE, bool SPH>
+static hipError_t launch_stage_end_mode(const StageArgs &a, hipStream_t st) {
+    const long n = long(a.nblk) * a.S;
+    const dim3 grid(unsigned((n + 63) / 64)), blk(64 * GW);     // 64 columns per workgroup
+    if (a.variant == 1) hipLaunchKernelGGL((k_stage_end<NSP, MODE, SPH, 4>), grid, blk, 0, st, a);
+    else hipLaunchKernelGGL((k_stage_end<NSP, MODE, SPH>), grid, blk, 0, st, a);
+    return hipGetLastError();
+}
+
 template <int NSP>
 static hipError_t launch_stage_end_nsp(const StageArgs &a, hipStream_t st) {
-    const long n = long(a.nblk) * a.S;
-    const int bs = a.variant == 2 ? 128 : (a.variant == 3 ? 256 : 64);
-    const dim3 grid(unsigned((n + bs - 1) / bs)), blk(bs);
-    switch (a.variant) {
-        case 1: hipLaunchKernelGGL((k_stage_end<NSP, 64, 1>), grid, blk, 0, st, a); break;
-        case 2: hipLaunchKernelGGL((k_stage_end<NSP, 128, 1>), grid, blk, 0, st, a); break;
-        case 3: hipLaunchKernelGGL((k_stage_end<NSP, 256, 1>), grid, blk, 0, st, a); break;
-        default: hipLaunchKernelGGL((k_stage_end<NSP>), grid, blk, 0, st, a); break;
-    }
-    return hipGetLastError();
+    if (a.mode == 2) return launch_stage_end_mode<NSP, 2, false>(a, st);
+    if (a.spherical) return a.mode == 0 ? launch_stage_end_mode<NSP, 0, true>(a, st) : launch_stage_end_mode<NSP, 1, true>(a, st);
+    return a.mode == 0 ? launch_stage_end_mode<NSP, 0, false>(a, st) : launch_stage_end_mode<NSP, 1, false>(a, st);
 }
 
 hipError_t launch_stage_end(const StageArgs &a, int nsp, hipStream_t st) {

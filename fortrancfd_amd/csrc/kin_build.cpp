@@ -1,4 +1,5 @@
 // kin_build.cpp -- device kinetics tables from the CHEMKIN-II link-file data (host side).
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -124,8 +125,25 @@ void build_dev_kin(const Mech &m, DevKin &k) {
     }
 }
 
-// CKHMS(298.15) (cklib.f:3598-3618): formation enthalpies for the heat-release diagnostics.
-void thermo_h298(DevThermo &t) {
+// Values that follow from the tables: CKHMS(298.15) (cklib.f:3598-3618), the formation enthalpies of
+// the heat-release diagnostics; 1 / wt; the coefficient sets by temperature class.
+void thermo_derived(DevThermo &t) {
+    for (int k = 0; k < t.kk; ++k) t.rwt[k] = 1.0 / t.wt[k];
+    const int M = (t.kk + SPECIES_BLOCKS - 1) / SPECIES_BLOCKS;
+    for (int w = 0; w < SPECIES_BLOCKS; ++w) {
+        const int k0 = std::min(w * M, t.kk), k1 = std::min(k0 + M, t.kk);
+        std::vector<double> cut(t.tmid + k0, t.tmid + k1);
+        std::sort(cut.begin(), cut.end());
+        cut.erase(std::unique(cut.begin(), cut.end()), cut.end());
+        t.nclass[w] = int(cut.size()) < MAXCLS ? int(cut.size()) + 1 : 0;
+        for (int c = 0; c < t.nclass[w]; ++c) {
+            if (c > 0) t.cut[w][c - 1] = cut[c - 1];
+            for (int k = k0; k < k1; ++k) {
+                const bool up = c > 0 && cut[c - 1] >= t.tmid[k];      // T > cut[c - 1] >= tmid
+                for (int i = 0; i < 6; ++i) t.coef[w][c][k - k0][i] = up ? t.ahi[k][i] : t.alo[k][i];
+            }
+        }
+    }
     const double T = 298.15, rut = T * t.ru;
     const double t2 = T * T, t3 = T * t2, t4 = t2 * t2;
     const double tn1 = T / 2.0, tn2 = t2 / 3.0, tn3 = t3 / 4.0, tn4 = t4 / 5.0;

@@ -136,7 +136,7 @@ int load_mech(const char *chem_bin, const char *tran_bin, Mech &m, std::string &
         }
     }
 
-    thermo_h298(d);
+    thermo_derived(d);
     return tran_bin ? load_tran_bin(tran_bin, m, err) : 0;
 }
 

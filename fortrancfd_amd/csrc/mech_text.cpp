@@ -479,7 +479,7 @@ thermo_tables:
                 d.ahi[k][c] = m.aa[(size_t(k) * 2 + 1) * 7 + c];
             }
         }
-        thermo_h298(d);
+        thermo_derived(d);
     }
     return 0;
 }

@@ -4,8 +4,8 @@ table that the library reads at start-up (fcfd_set_launch / fcfd_load_tuning).
     python -m fortrancfd_amd.tune [--out fortrancfd_amd/data/tuned_launch.txt] [--steps N]
 
 Candidates and the workloads they are timed on (GRI-3.0):
-  * flux_variant (WENO5 advection flux: 64 threads at two or one waves per SIMD, 128 threads) and
-    stage_variant (stage update: 64 / two, 64 / one, 128 / one, 256 / one) on inert hydrodynamics,
+  * flux_variant (WENO5 + HLLC advection flux) and stage_variant (stage update), the register budget
+    for three (0) or four (1) waves per SIMD, on inert hydrodynamics,
     64 blocks x 4096 cells, WENO5-JS + HLLC + SSP-RK3, kernel times from the context's HIP events;
   * chem_wg_per_cu (implicit-integrator workgroups per CU) on a long stiff list: 2^16 independent
     cells of the chemistry batch generator (fortrancfd_amd.workloads.chemistry_batch);
@@ -52,7 +52,7 @@ def tune_fluid(mech, log):
     nblk, ncell = 64, 4096
     cells = coupled_cells(mech, nblk, ncell, nhot=0)
     out = {}
-    for key, kid, cands in (("flux_variant", 0, (0, 1, 2)), ("stage_variant", 1, (0, 1, 2, 3))):
+    for key, kid, cands in (("flux_variant", 0, (0, 1)), ("stage_variant", 1, (0, 1))):
         res = {}
         for v in cands:
             set_launch(key, mech.kk, v)

@@ -223,9 +223,9 @@ int fcfd_set_timing(fcfd_ctx *c, int enable);
  * (python -m fortrancfd_amd.tune): data/tuned_launch.txt beside the library directory, or the file
  * FCFD_TUNE_FILE names; entries of other GPU architectures are ignored ("none" stands for a host
  * without a GPU), absent keys keep their
- * defaults.  Keys: "flux_variant" (WENO5 advection flux: 0 = 64 threads and two waves per SIMD,
- * 1 = 64 / one, 2 = 128 / one), "stage_variant" (stage update: 0 = 64 / two, 1 = 64 / one,
- * 2 = 128 / one, 3 = 256 / one), "chem_wg_per_cu" (implicit-integrator workgroups per CU, default 5),
+ * defaults.  Keys: "flux_variant" (WENO5 + HLLC advection flux: register budget for four waves
+ * per SIMD with 1, three with 0 or 2), "stage_variant" (stage update: four waves per SIMD with 1,
+ * three with 0, 2 or 3), "chem_wg_per_cu" (implicit-integrator workgroups per CU, default 5),
  * "chem_four_wave_factor" (four-wave integrator mode for lists of at most factor x workgroups cells,
  * default 8), "chem_lu" (how the four-wave integrator factors its Newton matrix: 0 = one elimination
  * step at a time through LDS, 1 = in 16-column panels with the FP64 matrix cores updating the rest,
