@@ -433,7 +433,7 @@ hipError_t enqueue_fluid(fcfd_ctx *c, double dt, const double *dt_dev) {
 
 hipError_t enqueue_dt(fcfd_ctx *c, double cfl, double *time_dev) {
     DtArgs a{};
-    a.thermo = c->thermo; a.qf = c->qf; a.cvel_bits = c->d_cvel; a.dt_out = c->d_dt; a.time = time_dev;
+    a.thermo = c->thermo; a.qf = c->qf; a.slots = c->d_cvel; a.dt_out = c->d_dt; a.time = time_dev;
     a.cfl = cfl; a.dx = c->dx; a.nblk = c->nblk; a.ncell = c->ncell; a.lv = c->lv; a.S = c->S; a.P = c->P;
     return timed(c, 2, [&]() { return launch_dt(a, c->kk, c->stream); });
 }
@@ -736,8 +736,8 @@ int create_impl(const fcfd_mech *m, const fcfd_opts *o, int nblk, int ncell, dou
     HIP_TRY(hipMemset(c->god, 0, sizeof(double) * 3 * c->PF));
     HIP_TRY(hipMalloc(&c->d_dt, sizeof(double)));
     HIP_TRY(hipMalloc(&c->d_time, sizeof(double)));
-    HIP_TRY(hipMalloc(&c->d_cvel, sizeof(unsigned long long)));
-    HIP_TRY(hipMemset(c->d_cvel, 0, sizeof(unsigned long long)));
+    HIP_TRY(hipMalloc(&c->d_cvel, DT_WORDS * sizeof(unsigned long long)));
+    HIP_TRY(hipMemset(c->d_cvel, 0, DT_WORDS * sizeof(unsigned long long)));
     HIP_TRY(hipMemset(c->d_dt, 0, sizeof(double)));
     if (!dxb.empty()) {
         c->h_dxb = dxb;

@@ -4,6 +4,8 @@
 // owns columns [b*S, (b+1)*S), S = ncell + 2*lv; its interior cell i (0-based) is column
 // b*S + lv + i, exactly the reference's b_obj(ib)%qf(:, ista-lv : iend+lv) column range.
 // Interface j (0..ncell) of block b -- the reference's Fplus(:, ista-1+j) -- is F[v*PF + b*(ncell+1)+j].
+#include <algorithm>
+
 #include "fluid_coop.hpp"
 #include "fluid.hpp"
 
@@ -519,50 +521,89 @@ __global__ void __launch_bounds__(64) k_smr_qf(SmrArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// calc_dt (SRC/update.f90:13-59): max wave speed over interior cells -> dt on the device.
+// calc_dt (SRC/update.f90:13-59): max wave speed over interior cells -> dt on the device.  64 cells
+// per workgroup of four waves, the species split over the waves as in k_stage_end; at most
+// 2048 workgroups, which stride over the cells; the last one to finish writes dt.  13 / 18 / 48 us for
+// 400 / 65,536 / 262,144 cells; one lane per cell and a launch of its own for dt took 18 / 25 / 53 us.
 // ---------------------------------------------------------------------------------------------
 template <int NSP>
-__global__ void __launch_bounds__(256) k_wave_speed(DtArgs a) {
-    const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    double aupc = 0.0;
-    if (t < long(a.nblk) * a.ncell) {
-        const int b = int(t / a.ncell), i = int(t % a.ncell);
-        const long c = long(b) * a.S + a.lv + i;
-        const DevThermo *__restrict__ m = a.thermo;
-        double x[NSP];
+__global__ void __launch_bounds__(64 * GW, 4) k_wave_speed(DtArgs a) {
+    constexpr int M = group_m<NSP>();
+    __shared__ CoopShared sh;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const unsigned n = unsigned(a.nblk) * unsigned(a.ncell);
+    CThermo *m = constant(a.thermo);
+    double most = 0.0;
+    for (unsigned t0 = blockIdx.x * 64u; t0 < n; t0 += gridDim.x * 64u) {
+        const unsigned t = min(t0 + unsigned(lane), n - 1u);      // a repeated cell changes no maximum
+        const unsigned b = t / unsigned(a.ncell), i = t - b * unsigned(a.ncell);
+        const unsigned cb = (b * unsigned(a.S) + unsigned(a.lv) + i) * 8u;
+        double y[M], x[M], s1[1];
+        bool ok = true;
 #pragma unroll
-        for (int k = 0; k < NSP; ++k) x[k] = a.qf[(3 + k) * a.P + c];
-        ytx<NSP>(m, x);                                   // no adjust_sum here (update.f90:396)
-        const double rho = a.qf[c], u = a.qf[a.P + c], T = a.qf[2 * a.P + c];
-        const double wtm = mix_w<NSP>(m, x);
-        const double p = (rho * 1.e-3) * m->ru * T / wtm * 0.1;
-        const MixSums ms = mix_sums<NSP>(m, x, T, false, true, true);
-        const double cp = ms.cpbml * 1.e-4 / wtm, cv = ms.cvbml * 1.e-4 / wtm;
-        const double as = sqrt(cp / cv * p / rho);
-        aupc = fmax(fmax(fabs(u - as), fabs(u)), fabs(u + as));
-    }
-    // wave64 max via cross-lane shuffles, then one LDS slot per wave
+        for (int j = 0; j < M; ++j) {
+            y[j] = at_byte(a.qf + long(3 + min(w * M + j, NSP - 1)) * a.P, cb);
+        }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) aupc = fmax(aupc, __shfl_xor(aupc, off, 64));
-    __shared__ double wmax[4];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) wmax[w] = aupc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double mx = wmax[0];
-        for (int k = 1; k < int(blockDim.x >> 6); ++k) mx = fmax(mx, wmax[k]);
-        // non-negative doubles order like their bit patterns
-        atomicMax(reinterpret_cast<unsigned long long *>(a.cvel_bits), (unsigned long long)__double_as_longlong(mx));
+        for (int j = 0; j < M; ++j) {
+            y[j] = w * M + j < NSP ? y[j] : 0.0;
+            ok = ok && num_ok(y[j]);
+        }
+        const double rho = at_byte(a.qf, cb), u = at_byte(a.qf + a.P, cb), T = at_byte(a.qf + 2 * a.P, cb);
+        const bool fast = __all(ok);
+        over_wt_coop<NSP>(m, w, fast, y, x);
+        chain_sum<1, M>(sh.c[0], w, lane, [&](int, int j) { return x[j]; }, s1);
+        ytx_coop<NSP>(m, w, fast, s1[0], y, x);                   // no adjust_sum here (update.f90:396)
+        double cp_k[M], unused[M], mix[3];
+        species_thermo<NSP, false, true>(m, w, T, __all(den_ok(T)), unused, cp_k);
+        const double ru = m->ru;
+        chain_sum<3, M>(sh.c[1], w, lane, [&](int c, int j) {
+            return x[j] * (c == 0 ? m->wt[min(w * M + j, NSP - 1)] : c == 1 ? cp_k[j] : cp_k[j] - ru);
+        }, mix);
+        if (w == 0) {
+            const double wtm = mix[0];
+            const double p = (rho * 1.e-3) * m->ru * T / wtm * 0.1;
+            const double cp = mix[1] * 1.e-4 / wtm, cv = mix[2] * 1.e-4 / wtm;
+            const double as = sqrt(cp / cv * p / rho);
+            most = fmax(most, fmax(fmax(fabs(u - as), fabs(u)), fabs(u + as)));
+        }
     }
-}
-
-__global__ void k_dt_finalize(DtArgs a) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        const double cvel = __longlong_as_double((long long)*a.cvel_bits);
-        const double dt = (a.cfl * a.dx) / cvel;
-        *a.dt_out = dt;
-        if (a.time) *a.time = *a.time + dt;
-        *a.cvel_bits = 0ull;
+    if (w == 0) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) most = fmax(most, __shfl_xor(most, off, 64));
+        // One address for every workgroup's maximum and arrival serialises them (1024 workgroups: 10 us);
+        // they meet at DT_SLOTS slots a cache line apart, and the last arrivals of the slots at one more.
+        // Non-negative doubles order like their bit patterns.  Everything passes through atomics, so
+        // no fence is needed (an agent-scope fence writes the L2 back, more than the whole kernel):
+        // each arrival only has to follow the atomic before it, whose returned value it takes in.
+        unsigned long long *slots = a.slots;
+        const unsigned g = blockIdx.x % DT_SLOTS, in_slot = (gridDim.x - g + DT_SLOTS - 1) / DT_SLOTS;
+        const unsigned nslots = min(gridDim.x, unsigned(DT_SLOTS));
+        int last = 0;
+        if (lane == 0) {
+            // (the sign bit of a maximum is 0)
+            const unsigned long long m0 = atomicMax(slots + g * 8, (unsigned long long)__double_as_longlong(most));
+            const unsigned long long n0 = atomicAdd(slots + g * 8 + 1, 1ull + (m0 >> 63));
+            if (n0 == in_slot - 1) last = atomicAdd(slots + DT_SLOTS * 8, 1ull) == nslots - 1;
+        }
+        if (__builtin_amdgcn_readfirstlane(last)) {
+            // the last workgroup of all: the maximum of the slots gives dt; every word is zero again
+            // for the next call
+            double cvel = 0.0;
+            if (unsigned(lane) < nslots) {
+                cvel = __longlong_as_double((long long)atomicExch(slots + lane * 8, 0ull));
+                atomicExch(slots + lane * 8 + 1, 0ull);
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) cvel = fmax(cvel, __shfl_xor(cvel, off, 64));
+            if (lane == 0) {
+                atomicExch(slots + DT_SLOTS * 8, 0ull);
+                const double dt = (a.cfl * a.dx) / cvel;
+                *a.dt_out = dt;
+                if (a.time) *a.time = *a.time + dt;
+            }
+        }
     }
 }
 
@@ -636,31 +677,63 @@ __global__ void k_qc_to_qf(const DevThermo *__restrict__ m, int n, const double 
 }
 
 // qfToQc on the interior columns of a padded domain (reaction_macks' final loop,
-// SRC/source.f90:78-82).
+// SRC/source.f90:78-82): 64 cells per workgroup of four waves, the species split as in k_stage_end
+// (18 us for 65,536 cells; 33 us with one lane per cell).
 template <int NSP>
-__global__ void __launch_bounds__(64) k_qf_to_qc_interior(const DevThermo *__restrict__ m, int nblk, int ncell, int lv, int S,
-                                    const double *__restrict__ qf, double *__restrict__ Qc, long P) {
-    const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= long(nblk) * ncell) return;
-    const long c = long(t / ncell) * S + lv + (t % ncell);
-    double y[NSP];
-    const double rho = qf[c], u = qf[P + c], T = qf[2 * P + c];
+__global__ void __launch_bounds__(64 * GW, 4) k_qf_to_qc_interior(const DevThermo *thermo, int nblk, int ncell, int lv,
+                                                                  int S, const double *qf, double *Qc, long P) {
+    constexpr int M = group_m<NSP>();
+    __shared__ CoopShared sh;
+    CThermo *m = constant(thermo);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const unsigned n = unsigned(nblk) * unsigned(ncell);
+    const unsigned t0 = xcd_block() * 64u + unsigned(lane);
+    const bool live = t0 < n;
+    const unsigned t = live ? t0 : n - 1u;
+    const unsigned b = t / unsigned(ncell);
+    const unsigned cb = (b * unsigned(S) + unsigned(lv) + (t - b * unsigned(ncell))) * 8u;
+    auto put = [cb, live](double *row, double v) {
+        if (live) *reinterpret_cast<double *>(reinterpret_cast<char *>(row) + cb) = v;
+    };
+    double y[M], x[M], s1[1];
 #pragma unroll
-    for (int k = 0; k < NSP; ++k) y[k] = qf[(3 + k) * P + c];
-    double ya[NSP];
+    for (int j = 0; j < M; ++j) y[j] = at_byte(qf + long(3 + min(w * M + j, NSP - 1)) * P, cb);
+    const double rho = at_byte(qf, cb), u = at_byte(qf + P, cb), T = at_byte(qf + 2 * P, cb);
+    bool ok = true;
 #pragma unroll
-    for (int k = 0; k < NSP; ++k) ya[k] = y[k];
-    adjust_sum<NSP>(ya);
+    for (int j = 0; j < M; ++j) {
+        y[j] = w * M + j < NSP ? y[j] : 0.0;
+        ok = ok && num_ok(y[j]);
+    }
+    const bool fast = __all(ok);
+    // rho Y from adjust_sum(Y), X = adjust_sum(CKYTX(Y)) from the raw Y
+    double s2[2];
+    over_wt_coop<NSP>(m, w, fast, y, x);
+    chain_sum<2, M>(sh.c[0], w, lane, [&](int c, int j) { return c == 0 ? fmax(y[j], 0.0) : x[j]; }, s2);
+    ytx_coop<NSP>(m, w, fast, s2[1], y, x);
 #pragma unroll
-    for (int k = 0; k < NSP; ++k) Qc[(3 + k) * P + c] = rho * ya[k];
-    ytx<NSP>(m, y);
-    adjust_sum<NSP>(y);
-    const double wtm = mix_w<NSP>(m, y);
-    const MixSums ms = mix_sums<NSP>(m, y, T, true, false, false);
-    const double e = ms.ubml * 1.e-4 / wtm;
-    Qc[c] = rho;
-    Qc[P + c] = rho * u;
-    Qc[2 * P + c] = rho * (e + 0.5 * (u * u));
+    for (int j = 0; j < M; ++j) {
+        y[j] = fmax(y[j], 0.0);
+        x[j] = fmax(x[j], 0.0);
+    }
+    scale_coop<M>(fast, s2[0], y);
+#pragma unroll
+    for (int j = 0; j < M; ++j)
+        if (w * M + j < NSP) put(Qc + long(3 + w * M + j) * P, rho * y[j]);
+    chain_sum<1, M>(sh.c[1], w, lane, [&](int, int j) { return x[j]; }, s1);
+    scale_coop<M>(fast, s1[0], x);
+    double hu[M], unused[M];
+    species_thermo<NSP, true, false>(m, w, T, __all(den_ok(T)), hu, unused);
+    chain_sum<2, M>(sh.c[0], w, lane, [&](int c, int j) {
+        return x[j] * (c == 0 ? m->wt[min(w * M + j, NSP - 1)] : hu[j]);
+    }, s2);
+    if (w == 0) {
+        const double e = s2[1] * 1.e-4 / s2[0];
+        put(Qc, rho);
+        put(Qc + P, rho * u);
+        put(Qc + 2 * P, rho * (e + 0.5 * (u * u)));
+    }
 }
 
 __global__ void k_recon(int n, const double *__restrict__ s, double *__restrict__ out) {
@@ -777,16 +850,11 @@ hipError_t launch_rk4_stage(const StageArgs &a, int nsp, hipStream_t st) {
 
 hipError_t launch_dt(const DtArgs &a, int nsp, hipStream_t st) {
     const long n = long(a.nblk) * a.ncell;
-    const dim3 grid(unsigned((n + 255) / 256)), blk(256);
-    bool launched = false;
-#define FCFD_CASE(N) if (!launched && nsp == N) { hipLaunchKernelGGL((k_wave_speed<N>), grid, blk, 0, st, a); launched = true; }
+    const dim3 grid(unsigned(std::min<long>((n + 63) / 64, 2048))), blk(64 * GW);
+#define FCFD_CASE(N) if (nsp == N) { hipLaunchKernelGGL((k_wave_speed<N>), grid, blk, 0, st, a); return hipGetLastError(); }
     FCFD_FOR_EACH_NSP(FCFD_CASE)
 #undef FCFD_CASE
-    if (!launched) return hipErrorInvalidValue;
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(64), 0, st, a);
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_init(const InitArgs &a, int nsp, hipStream_t st) {
@@ -817,7 +885,7 @@ hipError_t launch_qc_to_qf(const DevThermo *m, int nsp, int n, const double *Qc,
 hipError_t launch_qf_to_qc_interior(const DevThermo *m, int nsp, int nblk, int ncell, int lv, int S,
                                     const double *qf, double *Qc, long P, hipStream_t st) {
     const long n = long(nblk) * ncell;
-    const dim3 grid(unsigned((n + 63) / 64)), blk(64);
+    const dim3 grid(unsigned((n + 63) / 64)), blk(64 * GW);
 #define FCFD_CASE(N) if (nsp == N) { hipLaunchKernelGGL((k_qf_to_qc_interior<N>), grid, blk, 0, st, m, nblk, ncell, lv, S, qf, Qc, P); return hipGetLastError(); }
     FCFD_FOR_EACH_NSP(FCFD_CASE)
 #undef FCFD_CASE

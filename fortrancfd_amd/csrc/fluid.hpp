@@ -37,10 +37,13 @@ struct StageArgs {
     long P, PF;
 };
 
+constexpr int DT_SLOTS = 32;                     // slots of the CFL maximum: (maximum, arrivals), 64 bytes apart
+constexpr int DT_WORDS = DT_SLOTS * 8 + 8;       // and the slots done
+
 struct DtArgs {
     const DevThermo *thermo;
     const double *qf;
-    unsigned long long *cvel_bits;
+    unsigned long long *slots;       // DT_WORDS words, zero between calls (k_wave_speed)
     double *dt_out;
     double *time;          // optional running time, advanced by dt
     double cfl, dx;
