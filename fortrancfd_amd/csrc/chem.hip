@@ -40,42 +40,6 @@ constexpr int LDJ = 65;   // LDS row stride of the Jacobian (odd in 64-bit words
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
-__device__ __forceinline__ double bcast(double v, int src) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
-    return __hiloint2double(hi, lo);
-}
-
-// One DPP move of a double (both halves with the same control); rows outside ROWMASK and lanes
-// without a source keep their own value.
-template <int CTRL, int ROWMASK = 0xF>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(v), __double2loint(v), CTRL, ROWMASK, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(v), __double2hiint(v), CTRL, ROWMASK, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-
-// As dpp_f64, but lanes without a source and rows outside ROWMASK read 0.
-template <int CTRL, int ROWMASK = 0xF>
-__device__ __forceinline__ double dpp_f64_or0(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWMASK, 0xF, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWMASK, 0xF, true);
-    return __hiloint2double(hi, lo);
-}
-
-// Sum over the wave, the same value in every lane: prefix sums within rows of 16 lanes (row_shr
-// 1/2/4/8), then row totals carried across rows (row_bcast 15 / 31), lane 63 broadcast.  The order
-// of the additions is fixed, so equal inputs give bitwise equal sums in every wave.
-__device__ __forceinline__ double wsum(double v) {
-    v = v + dpp_f64_or0<0x111>(v);
-    v = v + dpp_f64_or0<0x112>(v);
-    v = v + dpp_f64_or0<0x114>(v);
-    v = v + dpp_f64_or0<0x118>(v);
-    v = v + dpp_f64_or0<0x142, 0xA>(v);
-    v = v + dpp_f64_or0<0x143, 0xC>(v);
-    return bcast(v, 63);
-}
-
 // Largest value over the wave: row_shr 1/2/4/8 within each row of 16 lanes, then row_bcast 15 / 31
 // across rows; lane 63 ends with the maximum.  fmax returns one of its operands, so the result is
 // bitwise one of the inputs (NaN inputs are passed over).

@@ -13,6 +13,45 @@
 namespace fcfd {
 
 // ---------------------------------------------------------------------------------------------
+// Cross-lane moves and sums of doubles
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ double bcast(double v, int src) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
+    return __hiloint2double(hi, lo);
+}
+
+// One DPP move of a double (both halves with the same control); rows outside ROWMASK and lanes
+// without a source keep their own value.
+template <int CTRL, int ROWMASK = 0xF>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(v), __double2loint(v), CTRL, ROWMASK, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(v), __double2hiint(v), CTRL, ROWMASK, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
+// As dpp_f64, but lanes without a source and rows outside ROWMASK read 0.
+template <int CTRL, int ROWMASK = 0xF>
+__device__ __forceinline__ double dpp_f64_or0(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWMASK, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWMASK, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Sum over the wave, the same value in every lane: prefix sums within rows of 16 lanes (row_shr
+// 1/2/4/8), then row totals carried across rows (row_bcast 15 / 31), lane 63 broadcast.  The order
+// of the additions is fixed, so equal inputs give bitwise equal sums in every wave.
+__device__ __forceinline__ double wsum(double v) {
+    v = v + dpp_f64_or0<0x111>(v);
+    v = v + dpp_f64_or0<0x112>(v);
+    v = v + dpp_f64_or0<0x114>(v);
+    v = v + dpp_f64_or0<0x118>(v);
+    v = v + dpp_f64_or0<0x142, 0xA>(v);
+    v = v + dpp_f64_or0<0x143, 0xC>(v);
+    return bcast(v, 63);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Thermo (CKLIB semantics)
 // ---------------------------------------------------------------------------------------------
 // Temperature powers shared by all species at one T (cklib.f:1849-1852, 3537-3541).
@@ -39,6 +78,22 @@ __device__ __forceinline__ TPow tpow(double T, double ru) {
     p.tnh1 = T / 2.0; p.tnh2 = t2 / 3.0; p.tnh3 = t3 / 4.0; p.tnh4 = t4 / 5.0;
     p.rtn0 = ru * 1.0; p.rtn1 = ru * T; p.rtn2 = ru * t2; p.rtn3 = ru * t3; p.rtn4 = ru * t4;
     return p;
+}
+
+// fm_exp for arguments inside the normal range of its result (|x| <= 700, where the bits are
+// fm_exp's): the power of two by one ldexp, no selects for special values.  Larger arguments are
+// clamped to +-1000 (infinity or 0).
+__device__ __forceinline__ double exp_core(double x) {
+    const double xc = __builtin_fmin(__builtin_fmax(x, -1000.0), 1000.0);
+    const double kd = (xc * FM_INV_LN2 + FM_SHIFT) - FM_SHIFT;
+    const double r0 = __builtin_fma(-kd, FM_LN2_HI, xc);
+    const double r1 = -kd * FM_LN2_LO;               // fm_exp's xl - kd * FM_LN2_LO with xl = 0
+    const double rh = r0 + r1;
+    const double rl = r1 - (rh - r0);
+    const double q = (rh * rh) * fm_exp_series(rh);
+    const double s = 1.0 + rh;
+    const double e = rh - (s - 1.0);
+    return __builtin_amdgcn_ldexp(s + (e + (rl + (rh * rl + q))), int(kd));
 }
 
 struct Nasa {

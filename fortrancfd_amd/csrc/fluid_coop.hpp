@@ -151,12 +151,12 @@ __device__ __forceinline__ double h_mol_r(const Nasa &a, const TPow &p, double r
     return p.rut * (s + quot(a.a5, p.T, rT));
 }
 
-// Molar u (erg/mol) and cp (erg/(mol K)) of the wave's species at the lanes' temperatures T (fast:
+// Molar u (with H: h; erg/mol) and cp (erg/(mol K)) of the wave's species at the lanes' temperatures T (fast:
 // every T of the wave in den_ok's range).  One pass per temperature class among the lanes, nearly
 // always one, two or three where a flame front crosses the wave: the class's coefficients are
 // scalar operands.  Selected per lane they cost 24 moves and 12 selects a species, more than the
 // polynomials.
-template <int NSP, bool U, bool CP>
+template <int NSP, bool U, bool CP, bool H = false>
 __device__ __forceinline__ void species_thermo(CThermo *m, int w, double T, bool fast,
                                                double (&u)[group_m<NSP>()], double (&c)[group_m<NSP>()]) {
     constexpr int M = group_m<NSP>();
@@ -167,7 +167,7 @@ __device__ __forceinline__ void species_thermo(CThermo *m, int w, double T, bool
         const double rT = recip(T);
         auto one = [&](CCoef *b, double &uj, double &cj) {
             const Nasa a{b[0], b[1], b[2], b[3], b[4], b[5], 0.0};
-            if (U) uj = h_mol_r(a, p, rT) - p.rut;
+            if (U) uj = H ? h_mol_r(a, p, rT) : h_mol_r(a, p, rT) - p.rut;
             if (CP) cj = cp_mol(a, p);
         };
         // (rows past the last species: unused rows of the table)
@@ -204,7 +204,7 @@ __device__ __forceinline__ void species_thermo(CThermo *m, int w, double T, bool
             const bool up = T > m->tmid[k];
             const Nasa a{up ? hi[0] : lo[0], up ? hi[1] : lo[1], up ? hi[2] : lo[2], up ? hi[3] : lo[3],
                          up ? hi[4] : lo[4], up ? hi[5] : lo[5], 0.0};
-            if (U) u[j] = h_mol(a, p) - p.rut;
+            if (U) u[j] = H ? h_mol(a, p) : h_mol(a, p) - p.rut;
             if (CP) c[j] = cp_mol(a, p);
             __builtin_amdgcn_sched_barrier(0);     // a rare path: no registers for overlap
         }
@@ -270,6 +270,40 @@ __device__ __forceinline__ void over_wt_coop(CThermo *m, int w, bool fast,
     }
 }
 
+// temperature_con (SRC/thermo.f90:211-257) from the wave's mole fractions x, with wtm = sum x wt.  The four
+// waves iterate on the same values, so they take the same decisions and meet at the same barriers.
+// Its sums use sh.c[1], then sh.c[0] and sh.c[1] in turn: the caller's last sum went through sh.c[0].
+template <int NSP>
+__device__ __forceinline__ double temperature_coop(CThermo *m, CoopShared &sh, int w, int lane, double e,
+                                                   const double (&x)[group_m<NSP>()], double &wtm) {
+    constexpr int M = group_m<NSP>();
+    double s1[1];
+    chain_sum<1, M>(sh.c[1], w, lane, [&](int, int j) { return x[j] * m->wt[min(w * M + j, NSP - 1)]; }, s1);
+    wtm = s1[0];
+    const double spe = e * 1.e4 * wtm;
+    double T = 1000.0, f = 1.e30, dT = 1.e30;
+    const double ru_gas = m->ru;
+    for (int it = 0; it < 10; ++it) {
+        const bool go = fabs(f) >= fabs(spe) * 1.e-9 && fabs(dT) >= T * 1.e-6;
+        if (!__any(go)) break;
+        double tu[M], tc[M], s[2];
+        species_thermo<NSP, true, true>(m, w, T, true, tu, tc);       // 20 <= T <= 6000
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            tu[j] = x[j] * tu[j];
+            tc[j] = x[j] * (tc[j] - ru_gas);
+        }
+        chain_sum<2, M>(sh.c[it & 1], w, lane, [&](int c, int j) { return c == 0 ? tu[j] : tc[j]; }, s);
+        if (go) {
+            f = s[0] - spe;
+            dT = -f / s[1];
+            T = T + dT;
+            T = fmax(20.0, fmin(6000.0, T));
+        }
+    }
+    return T;
+}
+
 // QcToqf (SRC/eos.f90:49-83) of one column per lane by the workgroup's four waves: rho, rho u and
 // rho E in every wave, q the wave's rho Y (0 past the last species).  Gives u, T and the wave's
 // renormalised mass fractions (store_y(j, y), before the temperature iteration, so that they need no
@@ -304,31 +338,7 @@ __device__ __forceinline__ void qc_to_qf_coop(CThermo *m, CoopShared &sh, int w,
     for (int j = 0; j < M; ++j) x[j] = fmax(x[j], 0.0);
     chain_sum<1, M>(sh.c[0], w, lane, [&](int, int j) { return x[j]; }, s1);      // adjust_sum
     scale_coop<M>(fast, s1[0], x);
-    // temperature_con (SRC/thermo.f90:211-257); the four waves iterate on the same values, so they
-    // take the same decisions and meet at the same barriers
-    chain_sum<1, M>(sh.c[1], w, lane, [&](int, int j) { return x[j] * m->wt[min(w * M + j, NSP - 1)]; }, s1);
-    const double spe = e * 1.e4 * s1[0];
-    T = 1000.0;
-    double f = 1.e30, dT = 1.e30;
-    const double ru_gas = m->ru;
-    for (int it = 0; it < 10; ++it) {
-        const bool go = fabs(f) >= fabs(spe) * 1.e-9 && fabs(dT) >= T * 1.e-6;
-        if (!__any(go)) break;
-        double tu[M], tc[M], s[2];
-        species_thermo<NSP, true, true>(m, w, T, true, tu, tc);       // 20 <= T <= 6000
-#pragma unroll
-        for (int j = 0; j < M; ++j) {
-            tu[j] = x[j] * tu[j];
-            tc[j] = x[j] * (tc[j] - ru_gas);
-        }
-        chain_sum<2, M>(sh.c[it & 1], w, lane, [&](int c, int j) { return c == 0 ? tu[j] : tc[j]; }, s);
-        if (go) {
-            f = s[0] - spe;
-            dT = -f / s[1];
-            T = T + dT;
-            T = fmax(20.0, fmin(6000.0, T));
-        }
-    }
+    T = temperature_coop<NSP>(m, sh, w, lane, e, x, s1[0]);
 }
 
 }  // namespace fcfd
