@@ -153,10 +153,11 @@ def measured_traffic(workload, kernel):
     if not os.path.isfile(path):
         return None, None
     kernels = json.load(open(path))["kernels"]
-    short = kernel.split(" ")[0] + "<"
-    # every instantiation launched for the call (the integrator launches its one-wave and its
-    # four-wave kernel each time; the one whose mode does not match the list returns at once)
-    hits = [rec["read_bytes"] + rec["write_bytes"] for name, rec in kernels.items() if short in name]
+    short = kernel.split(" ")[0]
+    # every kernel launched for the call (the integrator launches its one-wave and its eight-wave
+    # kernel each time; the one whose mode does not match the list returns at once)
+    hits = [rec["read_bytes"] + rec["write_bytes"] for name, rec in kernels.items()
+            if short + "<" in name or short + "_coop<" in name]
     if not hits:
         return None, None
     return sum(hits), os.path.relpath(path, REPO)

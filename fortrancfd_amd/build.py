@@ -20,12 +20,15 @@ LIB = os.path.join(OUT_DIR, "libfcfd_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["api.hip", "fluid.hip", "chem.hip", "chem_lane.hip", "tran.hip", "aux.hip", "mlp.hip", "surrogate.hip", "mech_io.cpp", "mech_text.cpp", "kin_build.cpp"]
+SOURCES = ["api.hip", "fluid.hip", "chem.hip", "chem_coop.hip", "chem_lane.hip", "tran.hip", "aux.hip", "mlp.hip", "surrogate.hip", "mech_io.cpp", "mech_text.cpp", "kin_build.cpp"]
 
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-ffp-contract=off", "-Wall",
           f"-I{os.path.join(REPO, 'include')}", f"-I{CSRC}"]
 HIP_FLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-munsafe-fp-atomics"]
+# Per source: chem_coop.hip's command loop keeps what it needs in registers only while the compiler does
+# not move every coefficient of its exponentials and logarithms in front of the loop.
+EXTRA_FLAGS = {"chem_coop.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def build(verbose: bool = False) -> str:
@@ -36,7 +39,7 @@ def build(verbose: bool = False) -> str:
         obj = os.path.join(OUT_DIR, os.path.splitext(src)[0] + ".o")
         cmd = [HIPCC, *COMMON]
         if src.endswith(".hip"):
-            cmd += ["-x", "hip", *HIP_FLAGS]
+            cmd += ["-x", "hip", *HIP_FLAGS, *EXTRA_FLAGS.get(src, [])]
         cmd += ["-c", path, "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)

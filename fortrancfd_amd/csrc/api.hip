@@ -154,11 +154,18 @@ int ensure_dev_tables(const fcfd_mech *cm) {
     // the tables go into the mechanism only when every step succeeded; a failure frees what was made
     int ncu = 0;
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    DevBuf th, kin, counter;
+    DevBuf th, kin, counter, lists;
     HIP_TRY(hipMalloc(&th.p, sizeof(DevThermo)));
     HIP_TRY(hipMemcpy(th.p, &m->host.thermo, sizeof(DevThermo), hipMemcpyHostToDevice));
     auto k = std::make_unique<DevKin>();
     build_dev_kin(m->host, *k);
+    std::vector<unsigned> jac;
+    build_coop_lists(*k, jac);
+    if (!jac.empty()) {
+        HIP_TRY(hipMalloc(&lists.p, jac.size() * sizeof(unsigned)));
+        HIP_TRY(hipMemcpy(lists.p, jac.data(), jac.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+        k->coop_jac = static_cast<const unsigned *>(lists.p);
+    }
     HIP_TRY(hipMalloc(&kin.p, sizeof(DevKin)));
     HIP_TRY(hipMemcpy(kin.p, k.get(), sizeof(DevKin), hipMemcpyHostToDevice));
     HIP_TRY(hipMalloc(&counter.p, sizeof(unsigned int)));
@@ -166,7 +173,8 @@ int ensure_dev_tables(const fcfd_mech *cm) {
     m->d_thermo = static_cast<DevThermo *>(th.p);
     m->d_kin = kin.p;
     m->d_counter = static_cast<unsigned int *>(counter.p);
-    th.p = kin.p = counter.p = nullptr;
+    m->d_lists = lists.p;
+    th.p = kin.p = counter.p = lists.p = nullptr;
     m->device = dev;
     return FCFD_OK;
 }
@@ -175,9 +183,9 @@ int ensure_dev_tables(const fcfd_mech *cm) {
 // A text table of "<arch> <species count> <key> <value>" lines: by default data/tuned_launch.txt
 // next to the library's directory (FCFD_TUNE_FILE overrides), read once per process; entries for
 // other GPU architectures are ignored.  Keys: flux_variant, stage_variant (fluid.hpp),
-// chem_wg_per_cu (integrator workgroups per CU), chem_four_wave_factor (four-wave mode for lists of
-// at most factor x workgroups cells), chem_lu (the four-wave integrator's LU: 0 step by step through
-// LDS, 1 blocked with matrix-core updates, 2 with the matrix in registers).
+// chem_wg_per_cu (integrator workgroups per CU), chem_four_wave_factor (eight waves per cell for
+// lists of at most factor x workgroups cells; four when the key was named), chem_lu (kept for tables
+// that hold it: the factorisations it chose between gave the same bits, and one is left).
 struct TuneTable {
     std::mutex mu;
     bool loaded = false;
@@ -256,8 +264,6 @@ static int launch_default(const char *key) {
 int chem_coop_max(int n_workgroups, int nsp) {
     return tuned(nsp, "chem_four_wave_factor", launch_default("chem_four_wave_factor")) * n_workgroups;
 }
-
-int chem_lu_variant(int nsp) { return tuned(nsp, "chem_lu", launch_default("chem_lu")); }
 
 // Persistent grid size: one-wave workgroups per CU (default five, as many as the LDS of a CU holds)
 // times the CUs.
@@ -673,6 +679,7 @@ void fcfd_mech_free(fcfd_mech *m) {
     if (!m) return;
     (void)hipFree(m->d_thermo);
     (void)hipFree(m->d_kin);
+    (void)hipFree(m->d_lists);
     (void)hipFree(m->d_counter);
     (void)hipFree(m->d_list);
     (void)hipFree(m->d_list_n);

@@ -34,6 +34,23 @@ struct LaneEnt {
     double nu;
 };
 
+// ---- tables of the integrator that gives a cell eight waves (chem_coop.hip) ----
+constexpr int COOP_WAVES = 8;        // waves per cell
+constexpr int COOP_MAXR = 384;       // reactions: six waves of one row per lane
+constexpr int COOP_LIST = COOP_MAXR * 6 + 4 * 64 * 3;      // list entries, padding included
+constexpr int COOP_TB = 8;           // enhanced third bodies of a row
+constexpr int COOP_FAL = 32;         // fall-off rows: two lanes of a wave each
+constexpr int COOP_EMPTY = 63;       // species index of an empty slot (concentration 1, coefficient 0)
+constexpr unsigned CR_REV = 1, CR_ARR0 = 2;   // DevKin::coop_row[2]: reversible; B = E = 0
+constexpr unsigned CR_POW = 4;       // some |coefficient| is 2 or 3
+constexpr int CR_NUS = 4;            // bits 4-6: coefficient sum + 3
+constexpr unsigned JE_NONE = 0xffff;
+constexpr int COOP_JAC = 1024;       // steps of a wave
+// Doubles per rate array: a place for each row and one that stays 0.  The arrays of 1, 2 and 3 times the
+// rates start at COOP_AT(1), (2), (3) of one LDS array, which holds the fall-off terms in between.
+constexpr int COOP_Q = COOP_MAXR + 1;
+constexpr int COOP_AT(int m) { return m == 1 ? 0 : (m - 1) * COOP_Q + 2 * COOP_FAL; }
+
 // Reaction data in the form CKRATT / CKRATX / CKWYR consume it (cklib.f:6630-6993, 9107-9204),
 // re-indexed 0-based with one row per reaction.
 struct DevKin {
@@ -58,9 +75,39 @@ struct DevKin {
     int lane_ent0[(MAXR + LANE_CHUNK - 1) / LANE_CHUNK * LANE_NW + 1];
     LaneEnt lane_ent[MAXR * 6];
     LanePlain lane_plain[MAXR];         // rows nplain0 .. ii-1 (other entries unused)
+    // Packed rows of the eight-wave integrator: [0] species of slots 0-3, a byte each (COOP_EMPTY: none);
+    // [1] those of slots 4 and 5; [2] CR_* and the coefficients as four-bit two's complement in bits
+    // 8 + 4 slot; [3] third-body row + 1, fall-off row + 1 in the upper half.
+    unsigned coop_row[4][MAXR];
+    // Third bodies of a row: species, a byte each (COOP_EMPTY: none), and efficiency - 1 (0)
+    unsigned coop_tbk[COOP_TB / 4][MAXR];
+    double coop_tba[COOP_TB][MAXR];
+    // 1: the mechanism suits that integrator: at most COOP_MAXR rows, |coefficients| and their sums at
+    // most 3, no negative product coefficient, no gap before a filled slot, at most COOP_TB third bodies
+    // and COOP_FAL fall-off rows, constants that over() may divide by T's reciprocal.
+    int coop;
+    // Its sums as lists of terms.  Row blocks of 64 form four groups (block 0; every third block from
+    // 1, 2, 3), each with a partial sum; within one the terms stand in the order block, slot, row.
+    //   coop_sum (production rates): group g's terms of species k are sum_len[g][k] entries from
+    //   sum_off[g][k] on, both multiples of four (padded by terms of rate 0).  A row's rate times 1, 2
+    //   and 3 stands in LDS; an entry is the place in bits 3-14 and the coefficient's sign in bit 15
+    //   coop_split (creation, destruction): place and, in bit 15, product slot (magnitude as above)
+    alignas(8) unsigned short coop_sum[COOP_LIST];
+    alignas(8) unsigned short coop_split[COOP_LIST];
+    unsigned short sum_off[4][64], sum_len[4][64];          // of either list
+    //   coop_jac (Jacobian entries): wave w takes jac_steps[w] steps (a multiple of eight), step l of its
+    //   lane at [jac_off[w] + 512 (l / 8) + 8 lane + l mod 8].  Four neighbouring lanes work on one entry, lane mod 4 on its
+    //   group's partial sum; the sixteen entries of a wave end at the same step.  A step: slot *
+    //   COOP_MAXR + row of the derivative in bits 3-14 (6 * COOP_MAXR: none), the upper half of the
+    //   coefficient as a double in bits 16-31; or, where jac_end[w] has its bit set, the place r * kk + c
+    //   of the finished entry (JE_NONE: none).  A device buffer of the mechanism.
+    const unsigned *coop_jac;
+    int jac_steps[COOP_WAVES], jac_off[COOP_WAVES];
+    unsigned char jac_end[COOP_WAVES][COOP_JAC / 8];        // bit u of byte b: step 8 b + u
 };
 
-
+// Fills the eight-wave integrator's tables of k; jac receives coop_jac's contents.
+void build_coop_lists(DevKin &k, std::vector<unsigned> &jac);
 void build_dev_kin(const Mech &m, DevKin &k);
 
 // Per-cell integrator counters (optional output).
@@ -95,7 +142,7 @@ struct ChemArgs {
     int *route;                  // optional per-cell route: 2 explicit step over dt, 3 two explicit half
                                  // steps, 1 surrogate, 0 implicit (SDIRK) integrator
     int layout;                  // 0: domain, 1: batch
-    int coop_max;                // set by launch_chem: lists up to this length run four waves per cell
+    int coop_max;                // set by launch_chem: lists up to this length run eight waves per cell
     // optional (domain layout with stats): buffer of the list's capacity that receives the list
     // reordered with the cells whose previous integration took the most attempts first
     int *order;
@@ -108,11 +155,11 @@ struct ChemArgs {
     // optional (domain layout): f at the start state of each cell the explicit screen rejects,
     // [NSP + 1][ncells] (species, then T); k_chem_retry starts from it instead of evaluating it again
     double *f0;
-    int lu_blocked;              // set by launch_chem: the four-wave mode's LU (0 lu, 1 lu_blocked, 2 lu_regs)
 };
 
 // SDIRK integrator over all cells or over a work list (persistent grid): one cell per wave for long
-// lists, one cell per four-wave workgroup for short ones.
+// lists, one cell per eight-wave workgroup (launch_chem_coop) for short ones.
+hipError_t launch_chem_coop(const ChemArgs &a, int nsp, int nwg, hipStream_t st);
 hipError_t launch_chem(const ChemArgs &a, int nsp, int n_workgroups, hipStream_t st);
 // Lane-per-cell explicit screen over cells 0 .. ncells: accepted cells are final, the others are
 // appended to a.stiff (a.stiff_n must be zero before the launch).
@@ -121,13 +168,9 @@ hipError_t launch_chem_screen(const ChemArgs &a, int nsp, hipStream_t st);
 // a.coop_max: accepted cells are final, the others go to a.stiff (a.stiff_n must be zero before
 // the launch) and *a.retry_done = 1; a shorter list is copied to a.stiff unchanged, *a.retry_done = 0.
 hipError_t launch_chem_retry(const ChemArgs &a, int nsp, hipStream_t st);
-// Length up to which a stiff list runs four waves per cell in launch_chem.
-// Longest list that the four-wave integrator mode takes: the tuned factor (default 8) times the
+// Longest list that the eight-wave integrator mode takes: the tuned factor (default 8) times the
 // workgroup count (api.hip).
 int chem_coop_max(int n_workgroups, int nsp);
-// The four-wave integrator's LU (the tuned "chem_lu" entry, api.hip): 0 step by step through LDS,
-// 1 blocked with matrix-core trailing updates, 2 with the matrix in registers; the same factors.
-int chem_lu_variant(int nsp);
 hipError_t launch_zero_u32(unsigned *p, hipStream_t st);
 // *out = f * *in on the device (one thread), e.g. the half step of Strang splitting.
 hipError_t launch_scale_scalar(const double *in, double *out, double f, hipStream_t st);

@@ -1,6 +1,7 @@
 // kin_build.cpp -- device kinetics tables from the CHEMKIN-II link-file data (host side).
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstdint>
 #include <cstring>
 #include <vector>
@@ -122,6 +123,139 @@ void build_dev_kin(const Mech &m, DevKin &k) {
         k.ifop[f] = m.ifo[f];
         k.kfal[f] = m.kfl[f] - 1;
         for (int c = 0; c < 8 && c < m.nfar; ++c) k.fpar[f][c] = m.fpar[size_t(f) * m.nfar + c];
+    }
+}
+
+void build_coop_lists(DevKin &k, std::vector<unsigned> &jac) {
+    const int ii = k.ii, nb = (ii + 63) / 64;
+    bool fits = ii <= COOP_MAXR && k.kk < COOP_EMPTY && k.nfal <= COOP_FAL;
+    auto usual = [](double v) { return v == 0.0 || (std::fabs(v) >= 0x1p-700 && std::fabs(v) <= 0x1p60); };
+    for (int f = 0; f < k.nfal; ++f) fits = fits && usual(k.fpar[f][2]) && usual(k.fpar[f][6]);
+    for (int r = 0; r < ii; ++r) {
+        const int *nu = k.nu[r], *nk = k.nk[r];
+        fits = fits && usual(k.E[r]);
+        fits = fits && std::abs(k.nus[r]) <= 3 && nk[0] >= 0 && nk[3] >= 0 && (nk[1] >= 0 || nk[2] < 0) &&
+               (nk[4] >= 0 || nk[5] < 0) && (k.tb[r] < 0 || k.ntbs[k.tb[r]] <= COOP_TB);
+        bool pow = false;
+        unsigned w[4] = {0, 0, 0, 0};
+        for (int n = 0; n < 6; ++n) {
+            fits = fits && std::abs(nu[n]) <= 3 && (n < 3 || nu[n] >= 0) && (nk[n] >= 0 || nu[n] == 0);
+            pow = pow || std::abs(nu[n]) > 1;
+            w[n / 4] |= unsigned(nk[n] >= 0 ? nk[n] : COOP_EMPTY) << (8 * (n % 4));
+            w[2] |= (unsigned(nu[n]) & 15u) << (8 + 4 * n);
+        }
+        w[2] |= (k.rev[r] ? CR_REV : 0u) | (k.arr0[r] ? CR_ARR0 : 0u) | (pow ? CR_POW : 0u) |
+                (unsigned(k.nus[r] + 3) & 7u) << CR_NUS;
+        w[3] = unsigned(k.tb[r] + 1) | unsigned(k.fo[r] + 1) << 16;
+        for (int n = 0; n < 4; ++n) k.coop_row[n][r] = w[n];
+        const int t = k.tb[r];
+        for (int l = 0; l < COOP_TB; ++l) {
+            const bool on = t >= 0 && l < k.ntbs[t];
+            if (l % 4 == 0) k.coop_tbk[l / 4][r] = 0;
+            k.coop_tbk[l / 4][r] |= unsigned(on ? std::max(k.tbk[t][l], 0) : COOP_EMPTY) << (8 * (l % 4));
+            k.coop_tba[l][r] = on ? k.tba[t][l] - 1.0 : 0.0;
+        }
+    }
+    k.coop = fits ? 1 : 0;
+    if (!fits) return;
+    auto group = [](int b) { return b == 0 ? 0 : 1 + (b - 1) % 3; };
+    // production rates, and the creation / destruction split
+    auto place = [](int r, int nu) {
+        const int m = std::abs(nu);
+        return (unsigned short)((m == 0 ? COOP_MAXR : COOP_AT(m) + r) << 3);
+    };
+    const unsigned short pad = place(0, 0);
+    int at = 0;
+    for (int g = 0; g < 4; ++g) {
+        std::vector<std::vector<unsigned short>> sum(64), split(64);
+        for (int b = 0; b < nb; ++b) {
+            if (group(b) != g) continue;
+            const int r0 = b * 64, r1 = std::min(ii, r0 + 64);
+            for (int n = 0; n < 6; ++n)
+                for (int r = r0; r < r1; ++r)
+                    if (k.nk[r][n] >= 0) sum[k.nk[r][n]].push_back((unsigned short)(place(r, k.nu[r][n]) | (k.nu[r][n] < 0 ? 0x8000 : 0)));
+            for (int n = 0; n < 3; ++n)
+                for (int half = 0; half < 2; ++half)
+                    for (int r = r0; r < r1; ++r) {
+                        const int s = n + 3 * half;
+                        if (k.nk[r][s] >= 0)
+                            split[k.nk[r][s]].push_back((unsigned short)(place(r, k.nu[r][s]) | half << 15));
+                    }
+        }
+        for (int s = 0; s < 64; ++s) {
+            while (sum[s].size() % 4) {
+                sum[s].push_back(pad);
+                split[s].push_back(pad);
+            }
+            k.sum_off[g][s] = (unsigned short)at;
+            k.sum_len[g][s] = (unsigned short)sum[s].size();
+            for (size_t e = 0; e < sum[s].size(); ++e, ++at) {
+                k.coop_sum[at] = sum[s][e];
+                k.coop_split[at] = split[s][e];
+            }
+        }
+    }
+    // Jacobian entries d(wdot_r) / d(c_c) = sum nu[t] dq[s] over slots t holding r and s holding c
+    auto upper16 = [](int v) {
+        const double d = v;
+        uint64_t b;
+        std::memcpy(&b, &d, sizeof b);
+        return unsigned(b >> 32) & 0xffff0000u;      // (small whole numbers: all other bits are 0)
+    };
+    struct Entry { unsigned dst; std::vector<unsigned> e[4]; size_t steps; };
+    std::vector<Entry> all(size_t(k.kk) * k.kk);
+    for (int b = 0; b < nb; ++b)
+        for (int s = 0; s < 6; ++s)
+            for (int t = 0; t < 6; ++t)
+                for (int r = b * 64; r < std::min(ii, b * 64 + 64); ++r) {
+                    if (k.nu[r][0] == 0 || k.nk[r][s] < 0 || k.nk[r][t] < 0) continue;
+                    all[size_t(k.nk[r][t]) * k.kk + k.nk[r][s]].e[group(b)].push_back(
+                        unsigned(s * COOP_MAXR + r) << 3 | upper16(k.nu[r][t]));
+                }
+    std::vector<Entry> entries;
+    for (size_t i = 0; i < all.size(); ++i) {
+        all[i].dst = unsigned(i);
+        all[i].steps = 0;
+        for (auto &g : all[i].e) all[i].steps = std::max(all[i].steps, g.size());
+        if (all[i].steps) entries.push_back(all[i]);
+    }
+    std::stable_sort(entries.begin(), entries.end(), [](const Entry &a, const Entry &b) { return a.steps > b.steps; });
+    // Rounds of sixteen entries, longest first, each to the wave with the fewest steps so far.  Waves 1 ..
+    // 4 also add up the production rates before: they start with those steps' share.
+    constexpr unsigned none = unsigned(6 * COOP_MAXR) << 3;
+    std::vector<std::vector<unsigned>> lane(COOP_WAVES * 64);
+    size_t load[COOP_WAVES];
+    for (int w = 0; w < COOP_WAVES; ++w) {
+        load[w] = 0;
+        if (w >= 1 && w <= 4)
+            for (int s = 0; s < 64; ++s) load[w] = std::max(load[w], size_t(k.sum_len[w - 1][s]));
+    }
+    std::vector<size_t> ends[COOP_WAVES];
+    for (size_t e0 = 0; e0 < entries.size(); e0 += 16) {
+        const int w = int(std::min_element(load, load + COOP_WAVES) - load);
+        const size_t steps = entries[e0].steps;
+        load[w] += steps + 2;
+        for (int i = 0; i < 16; ++i) {
+            const Entry *en = e0 + i < entries.size() ? &entries[e0 + i] : nullptr;
+            for (int g = 0; g < 4; ++g) {
+                std::vector<unsigned> &l = lane[w * 64 + i * 4 + g];
+                for (size_t e = 0; e < steps; ++e) l.push_back(en && e < en->e[g].size() ? en->e[g][e] : none);
+                l.push_back(en ? en->dst : JE_NONE);
+            }
+        }
+        ends[w].push_back(lane[w * 64].size() - 1);
+    }
+    for (int w = 0; w < COOP_WAVES; ++w) {
+        const size_t mx = std::max<size_t>((lane[w * 64].size() + 7) / 8 * 8, 8);      // the kernel loads eight steps at a time
+        k.coop = k.coop && mx <= COOP_JAC ? 1 : 0;
+        if (!k.coop) return;
+        k.jac_steps[w] = int(mx);
+        k.jac_off[w] = int(jac.size());
+        std::memset(k.jac_end[w], 0, sizeof k.jac_end[w]);
+        for (size_t e : ends[w]) k.jac_end[w][e / 8] |= (unsigned char)(1u << (e % 8));
+        jac.resize(jac.size() + mx * 64, none);
+        for (int i = 0; i < 64; ++i)
+            for (size_t e = 0; e < lane[w * 64 + i].size(); ++e) jac[k.jac_off[w] + e / 8 * 512 + i * 8 + e % 8] = lane[w * 64 + i][e];
     }
 }
 

@@ -9,11 +9,10 @@ Candidates and the workloads they are timed on (GRI-3.0):
     64 blocks x 4096 cells, WENO5-JS + HLLC + SSP-RK3, kernel times from the context's HIP events;
   * chem_wg_per_cu (implicit-integrator workgroups per CU) on a long stiff list: 2^16 independent
     cells of the chemistry batch generator (fortrancfd_amd.workloads.chemistry_batch);
-  * chem_four_wave_factor (the list length below which the integrator gives each cell four waves)
-    and chem_lu (the four-wave mode's LU: step by step through LDS, in 16-column panels with the
-    FP64 matrix cores, or with the matrix in registers; the factors are bitwise the same) on whole
-    steps of the coupled 65536-cell domain: the run continued for 200 steps from its state after
-    --steps Strang steps, per candidate (chem_lu first, at the default factor).
+  * chem_four_wave_factor (the list length up to which the integrator gives each cell a workgroup of
+    its own, eight waves; the key dates from when it was four) on whole steps of the coupled
+    65536-cell domain: the run continued for 200 steps from its state after --steps Strang steps, per
+    candidate.
 A candidate replaces the default only when it is more than 2 % faster.
 Each candidate is timed three times and scored by its median; the table records the winners and,
 as comments, every candidate's time.
@@ -105,7 +104,7 @@ def tune_chem_long(mech, log, n=1 << 16):
 
 
 def tune_chem_short(mech, log, steps, window=200):
-    """chem_four_wave_factor and chem_lu on whole coupled steps: the coupled 65536-cell domain
+    """chem_four_wave_factor on whole coupled steps: the coupled 65536-cell domain
     (Strang, HRR every step) run to `steps`, then `window` steps from that saved state per candidate
     (ms per step, median of three).  The window takes in the stiff lists of every length the run
     produces -- the short lists of the hot spots and the periodic bursts of a thousand or more cold
@@ -128,23 +127,14 @@ def tune_chem_short(mech, log, steps, window=200):
             reps.append((time.perf_counter() - t0) * 1e3 / window)
         return median(reps)
 
-    # the four-wave mode's factorisation first (step by step through LDS, blocked on the matrix
-    # cores, or in registers: the same factors), at the default factor
-    lu = {}
-    for v in (0, 1, 2):
-        set_launch("chem_lu", mech.kk, v)
-        lu[v] = per_step()
-        log(f"chem_lu={v}: {lu[v]:.3f} ms per coupled step (four-wave factor 8)")
-    best_lu = pick(lu, 2)
-    set_launch("chem_lu", mech.kk, best_lu)
     res = {}
     for v in (0, 1, 2, 4, 8):
         set_launch("chem_four_wave_factor", mech.kk, v)
         res[v] = per_step()
-        log(f"chem_four_wave_factor={v}: {res[v]:.3f} ms per coupled step (steps {steps}-{steps + window}, chem_lu {best_lu})")
+        log(f"chem_four_wave_factor={v}: {res[v]:.3f} ms per coupled step (steps {steps}-{steps + window})")
     best = pick(res, 8)
     set_launch("chem_four_wave_factor", mech.kk, best)
-    return best, res, best_lu
+    return best, res
 
 
 def main(argv=None):
@@ -163,17 +153,15 @@ def main(argv=None):
         lines.append("# " + msg)
 
     # start from the defaults, whatever table is installed
-    for key, v in (("flux_variant", 0), ("stage_variant", 0), ("chem_wg_per_cu", 5), ("chem_four_wave_factor", 8),
-                   ("chem_lu", 2)):
+    for key, v in (("flux_variant", 0), ("stage_variant", 0), ("chem_wg_per_cu", 5), ("chem_four_wave_factor", 8)):
         set_launch(key, mech.kk, v)
     fl = tune_fluid(mech, log)
     wg, _ = tune_chem_long(mech, log)
-    fw, _, lu = tune_chem_short(mech, log, args.steps)
+    fw, _ = tune_chem_short(mech, log, args.steps)
     table = [f"{arch} {mech.kk} flux_variant {fl['flux_variant'][0]}",
              f"{arch} {mech.kk} stage_variant {fl['stage_variant'][0]}",
              f"{arch} {mech.kk} chem_wg_per_cu {wg}",
-             f"{arch} {mech.kk} chem_four_wave_factor {fw}",
-             f"{arch} {mech.kk} chem_lu {lu}"]
+             f"{arch} {mech.kk} chem_four_wave_factor {fw}"]
     with open(args.out, "w") as f:
         f.write("# Launch shapes chosen by python -m fortrancfd_amd.tune (median of three timings each).\n")
         f.write("# Lines: <arch> <species count> <key> <value>; read by libfcfd_hip.so at start-up.\n")
