@@ -1,31 +1,18 @@
-// mlp.hip -- kernels of the chemistry surrogate (forward, backward, Adam, feature / target
-// construction, and the inference epilogue that decides between the surrogate and the FP64
-// integrator for each cell).
+// mlp.hip -- kernels around the chemistry surrogate's network (mlp_net.hip): feature / target construction,
+// batch gathering, the loss, the inference epilogue that decides between the surrogate and the FP64
+// integrator for each cell, and a plain BF16 GEMM.
 //
 // GEMM: C[M x N] = A[M x K] * B[K x N] in BF16 with FP32 accumulation on v_mfma_f32_16x16x16bf16_1k.
 // A workgroup of 4 waves owns a 64 x 64 tile of C (each wave 32 x 32 = 2 x 2 MFMA blocks); the K loop
 // stages a 64 x 16 slice of A and a 16 x 64 slice of B in LDS (B stored n-major so each lane's
-// 4-element fragment is one 8-byte read).  Operands are addressed through (row, col) strides, so
-// the same kernel serves X*W (forward), dPre*W^T (backward data) and H^T*dPre (backward weights,
-// split over K into partial buffers reduced in a fixed order).
+// 4-element fragment is one 8-byte read).  Operands are addressed through (row, col) strides.
 #include <cmath>
 
-#include "fcfd_device.hpp"
 #include "mlp.hpp"
+#include "mlp_device.hpp"
 #include "surrogate.hpp"
 
 namespace fcfd {
-
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint16_t f2bf(float f) {        // round to nearest even
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u) return uint16_t(u >> 16) | ((u & 0xffffu) ? 0x40 : 0);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return uint16_t(u >> 16);
-}
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(uint32_t(h) << 16); }
 
 // Box-Cox transform of a mass fraction, lambda = 1/10: b(Y) = 10 (Y^0.1 - 1), b(0) = -10, and its
 // inverse Y = (b / 10 + 1)^10 (0 where the base is not positive).
@@ -37,11 +24,6 @@ __device__ __forceinline__ double boxcox_inv(double b) {
     return v8 * v2;
 }
 
-__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_d(float x) {
-    return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
-}
-
 // ---------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs a) {
     __shared__ uint16_t As[64][16 + 4];
@@ -50,12 +32,6 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs a) {
     const int tiles_n = a.N / 64;
     const int tile = blockIdx.x;
     const int m0 = (tile / tiles_n) * 64, n0 = (tile % tiles_n) * 64;
-    if (a.m_dev && a.m_off + m0 >= int(*a.m_dev)) return;   // uniform per workgroup, before any barrier
-    if (a.m_dev && a.row_live) {
-        // every wave reads the same 64 flags, so all four leave together, before any barrier
-        const int r = a.m_off + m0 + lane;
-        if (!__any(r < int(*a.m_dev) && a.row_live[r] != 0)) return;
-    }
     const int split = blockIdx.y;
     const int kchunk = a.K / a.ksplit;
     const int kbeg = split * kchunk, kend = kbeg + kchunk;
@@ -101,18 +77,7 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs a) {
                 const int m = m0 + wm + i * 16 + (lane >> 4) * 4 + q;
                 const int n = n0 + wn + j * 16 + (lane & 15);
                 const long o = long(m) * a.ldc + n;
-                const float v = acc[i][j][q];
-                switch (a.epilogue) {
-                    case EP_STORE: a.C32[long(split) * a.M * a.ldc + o] = v; break;
-                    case EP_BIAS: a.C32[o] = v + a.bias[n]; break;
-                    case EP_BIAS_GELU: {
-                        const float p = v + a.bias[n];
-                        if (a.P32) a.P32[o] = p;
-                        a.C16[o] = f2bf(gelu(p));
-                        break;
-                    }
-                    default: a.C16[o] = f2bf(v * gelu_d(a.P32[o])); break;
-                }
+                a.C32[long(split) * a.M * a.ldc + o] = acc[i][j][q];
             }
 }
 
@@ -236,56 +201,22 @@ __global__ void __launch_bounds__(256) k_mse(const float *Yh, const float *Yt, u
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// out[j] = sum_s parts[s*len + j] (fixed order).
-__global__ void k_reduce_splits(const float *parts, float *out, int nsplit, long len) {
-    const long j = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= len) return;
-    float s = 0.f;
-    for (int q = 0; q < nsplit; ++q) s += parts[q * len + j];
-    out[j] = s;
-}
-
-// Column sums of a BF16 matrix (bias gradients), first stage: partial[chunk][j] over 64-row chunks.
-__global__ void k_colsum(const uint16_t *D, float *partial, int rows, int cols) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int chunk = blockIdx.y;
-    if (j >= cols) return;
-    float s = 0.f;
-    const int r1 = min(rows, (chunk + 1) * 64);
-    for (int r = chunk * 64; r < r1; ++r) s += bf2f(D[long(r) * cols + j]);
-    partial[long(chunk) * cols + j] = s;
-}
-
 __global__ void k_zero_u32(unsigned *p) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0u;
 }
 
-__global__ void k_sum_partials(const float *p, int n, float *out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        float s = 0.f;
-        for (int i = 0; i < n; ++i) s += p[i];
-        *out = s;
+// Sum of n values: one workgroup, strided partial sums and a tree.
+__global__ void __launch_bounds__(256) k_sum_partials(const float *p, int n, float *out) {
+    __shared__ float red[256];
+    float s = 0.f;
+    for (int i = threadIdx.x; i < n; i += 256) s += p[i];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+        if (threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+        __syncthreads();
     }
-}
-
-// Adam on FP32 master parameters; refreshes the BF16 copies of weights (w16 may be null for biases).
-__global__ void k_adam(float *w, const float *g, float *m, float *v, uint16_t *w16, long n, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
-    const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    w[i] = wi;
-    if (w16) w16[i] = f2bf(wi);
-}
-
-__global__ void k_to_bf16(const float *w, uint16_t *w16, long n) {
-    const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) w16[i] = f2bf(w[i]);
+    if (threadIdx.x == 0) *out = red[0];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -456,35 +387,12 @@ hipError_t mlp_mse(const float *Yh, const float *Yt, uint16_t *dY, int rows, flo
                    hipStream_t st) {
     const unsigned nb = blocks(long(rows) * MLP_OUTP, 256);
     hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, st, Yh, Yt, dY, rows, partial);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(64), 0, st, partial, int(nb), loss);
-    return hipGetLastError();
-}
-
-hipError_t mlp_reduce_splits(const float *parts, float *out, int nsplit, long len, hipStream_t st) {
-    hipLaunchKernelGGL(k_reduce_splits, dim3(blocks(len, 256)), dim3(256), 0, st, parts, out, nsplit, len);
-    return hipGetLastError();
-}
-
-hipError_t mlp_colsum(const uint16_t *D, float *partial, float *out, int rows, int cols, hipStream_t st) {
-    const int nchunk = (rows + 63) / 64;
-    hipLaunchKernelGGL(k_colsum, dim3(blocks(cols, 64), unsigned(nchunk)), dim3(64), 0, st, D, partial, rows, cols);
-    hipLaunchKernelGGL(k_reduce_splits, dim3(blocks(cols, 256)), dim3(256), 0, st, partial, out, nchunk, long(cols));
+    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, st, partial, int(nb), loss);
     return hipGetLastError();
 }
 
 hipError_t mlp_zero_u32(unsigned *p, hipStream_t st) {
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, p);
-    return hipGetLastError();
-}
-
-hipError_t mlp_adam(float *w, const float *g, float *m, float *v, uint16_t *w16, long n, float lr, float b1, float b2,
-                    float eps, float c1, float c2, hipStream_t st) {
-    hipLaunchKernelGGL(k_adam, dim3(blocks(n, 256)), dim3(256), 0, st, w, g, m, v, w16, n, lr, b1, b2, eps, c1, c2);
-    return hipGetLastError();
-}
-
-hipError_t mlp_to_bf16(const float *w, uint16_t *w16, long n, hipStream_t st) {
-    hipLaunchKernelGGL(k_to_bf16, dim3(blocks(n, 256)), dim3(256), 0, st, w, w16, n);
     return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
 // surrogate.hip -- host side of the chemistry surrogate: parameter and workspace management,
-// the forward / backward / Adam sequence of one training step, batched inference with FP64
+// the forward / backward / update sequence of one training step, batched inference with FP64
 // fallback, and the surrogate branch of solve_source.  All work is stream-ordered and
 // allocation-free once the workspace is sized, so a solve_source with the surrogate can be
 // captured in a HIP graph.
@@ -56,9 +56,6 @@ hipError_t Surrogate::reserve(int rows, bool training) {
     if ((e = grow(stiff, capST, r)) != hipSuccess) return e;
     if ((e = grow(cand_list, capCL, r)) != hipSuccess) return e;
     if ((e = grow(cand, capCD, r * size_t(mech->host.kk + 1))) != hipSuccess) return e;
-    const size_t hr = std::min<size_t>(r, size_t(INFER_CHUNK));
-    for (int i = 0; i < 2; ++i)
-        if ((e = grow(Hping[i], capH[i], hr * MLP_HID)) != hipSuccess) return e;
     if (!training) return hipSuccess;
     for (int l = 0; l < 4; ++l) {
         if ((e = grow(H[l], capHl[l], r * MLP_HID)) != hipSuccess) return e;
@@ -66,101 +63,77 @@ hipError_t Surrogate::reserve(int rows, bool training) {
     }
     if ((e = grow(Yt, capYt, r * MLP_OUTP)) != hipSuccess) return e;
     if ((e = grow(dY, capdY, r * MLP_OUTP)) != hipSuccess) return e;
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i)
         if ((e = grow(dZ[i], capdZ[i], r * MLP_HID)) != hipSuccess) return e;
-    if ((e = grow(cs_part, capCS, ((r + 63) / 64) * MLP_HID)) != hipSuccess) return e;
+    if ((e = grow(cs_part, capCS, ((r + 63) / 64) * (4 * MLP_HID + MLP_OUTP))) != hipSuccess) return e;
     if ((e = grow(loss_part, capLP, (r * MLP_OUTP + 255) / 256 + 1)) != hipSuccess) return e;
     return hipSuccess;
 }
 
-hipError_t Surrogate::gemm(const uint16_t *A, long sam, long sak, const uint16_t *B, long sbk, long sbn, int M,
-                           int N, int K, int ksplit, int ep, float *C32, uint16_t *C16, float *P32,
-                           const float *bias, long ldc, hipStream_t st, const unsigned *m_dev, int m_off,
-                           const int *row_live) const {
-    GemmArgs g{};
-    g.m_dev = m_dev;
-    g.m_off = m_off;
-    g.row_live = row_live;
-    g.A = A; g.B = B; g.sam = sam; g.sak = sak; g.sbk = sbk; g.sbn = sbn;
-    g.M = M; g.N = N; g.K = K; g.ksplit = ksplit;
-    g.C32 = C32; g.C16 = C16; g.P32 = P32; g.bias = bias; g.ldc = ldc; g.epilogue = ep;
-    return launch_gemm(g, st);
+NetParams Surrogate::params() const {
+    NetParams p{};
+    int f = 0, r = 0;
+    for (int l = 0; l < MLP_LAYERS; ++l) {
+        p.K[l] = MLP_K[l]; p.N[l] = MLP_N[l];
+        p.W[l] = W32[l]; p.b[l] = b32[l]; p.gW[l] = gW[l]; p.gb[l] = gb[l];
+        p.mW[l] = mW[l]; p.vW[l] = vW[l]; p.mb[l] = mb[l]; p.vb[l] = vb[l];
+        p.fwd0[l] = f;
+        f += int(wsize(l));
+    }
+    for (int l = MLP_LAYERS - 1; l > 0; --l) {
+        p.bwd0[l] = r;
+        r += int(wsize(l));
+    }
+    p.fwd = Wfwd; p.bwd = Wbwd;
+    return p;
 }
 
-// Forward of `rows` rows of X (rows multiple of 64).  Training keeps every layer's activations
-// and pre-activations; inference ping-pongs two activation buffers chunk by chunk.
+// Forward of `rows` rows of x (rows multiple of 64).  Training keeps every layer's activations and
+// pre-activations.
 hipError_t Surrogate::forward(const uint16_t *x, int rows, float *out, bool training, hipStream_t st,
                               const unsigned *m_dev, const int *row_live) {
-    hipError_t e;
-    if (training) {
-        const uint16_t *in = x;
-        for (int l = 0; l < 4; ++l) {
-            e = gemm(in, MLP_K[l], 1, W16[l], MLP_N[l], 1, rows, MLP_N[l], MLP_K[l], 1, EP_BIAS_GELU, nullptr, H[l],
-                     Pre[l], b32[l], MLP_N[l], st);
-            if (e != hipSuccess) return e;
-            in = H[l];
-        }
-        return gemm(in, MLP_HID, 1, W16[4], MLP_OUTP, 1, rows, MLP_OUTP, MLP_HID, 1, EP_BIAS, out, nullptr, nullptr,
-                    b32[4], MLP_OUTP, st);
-    }
-    for (int r0 = 0; r0 < rows; r0 += INFER_CHUNK) {
-        const int cr = std::min(INFER_CHUNK, rows - r0);
-        const uint16_t *in = x + long(r0) * MLP_INP;
-        for (int l = 0; l < 4; ++l) {
-            uint16_t *o = Hping[l & 1];
-            e = gemm(in, MLP_K[l], 1, W16[l], MLP_N[l], 1, cr, MLP_N[l], MLP_K[l], 1, EP_BIAS_GELU, nullptr, o,
-                     nullptr, b32[l], MLP_N[l], st, m_dev, r0, row_live);
-            if (e != hipSuccess) return e;
-            in = o;
-        }
-        e = gemm(in, MLP_HID, 1, W16[4], MLP_OUTP, 1, cr, MLP_OUTP, MLP_HID, 1, EP_BIAS, out + long(r0) * MLP_OUTP,
-                 nullptr, nullptr, b32[4], MLP_OUTP, st, m_dev, r0, row_live);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    NetArgs a{};
+    a.x = x; a.w = Wfwd; a.rows = rows; a.out = out;
+    a.wide = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+    a.m_dev = m_dev; a.row_live = row_live;
+    for (int l = 0; l < MLP_LAYERS; ++l) a.bias[l] = b32[l];
+    if (training)
+        for (int l = 0; l < 4; ++l) { a.H[l] = H[l]; a.P[l] = Pre[l]; }
+    return net_forward(a, training, st);
 }
 
-// Gradients of the mean squared error of the current batch (X, Yt already in place) into gW / gb.
-hipError_t Surrogate::backward(int rows, hipStream_t st) {
+hipError_t Surrogate::train(int rows, float lr, hipStream_t st) {
     hipError_t e;
     if ((e = forward(X, rows, Yh, true, st)) != hipSuccess) return e;
     if ((e = mlp_mse(Yh, Yt, dY, rows, loss_part, d_loss, st)) != hipSuccess) return e;
-    const uint16_t *dz = dY;
-    for (int l = MLP_LAYERS - 1; l >= 0; --l) {
-        const int K = MLP_K[l], N = MLP_N[l];
-        const uint16_t *hin = l == 0 ? X : H[l - 1];
-        const int tiles = (K / 64) * (N / 64);
-        const int ks = choose_split(rows, tiles);
-        if ((e = gemm(hin, 1, K, dz, N, 1, K, N, rows, ks, EP_STORE, gpart, nullptr, nullptr, nullptr, N, st)) !=
-            hipSuccess)
-            return e;
-        if ((e = mlp_reduce_splits(gpart, gW[l], ks, wsize(l), st)) != hipSuccess) return e;
-        if ((e = mlp_colsum(dz, cs_part, gb[l], rows, N, st)) != hipSuccess) return e;
-        if (l > 0) {
-            uint16_t *dn = dZ[l & 1];
-            if ((e = gemm(dz, N, 1, W16[l], 1, N, rows, K, N, 1, EP_GELU_BWD, nullptr, dn, Pre[l - 1], nullptr, K,
-                          st)) != hipSuccess)
-                return e;
-            dz = dn;
-        }
-    }
-    return hipSuccess;
-}
-
-hipError_t Surrogate::adam(float lr, hipStream_t st) {
-    ++step;
-    const float c1 = 1.0f - std::pow(ADAM_B1, float(step));
-    const float c2 = 1.0f - std::pow(ADAM_B2, float(step));
-    hipError_t e;
+    NetArgs a{};
+    a.x = dY; a.w = Wbwd; a.rows = rows; a.wide = 1;
+    for (int i = 0; i < 4; ++i) { a.H[i] = dZ[3 - i]; a.P[i] = Pre[3 - i]; }     // from the last hidden layer down
+    if ((e = net_backward(a, st)) != hipSuccess) return e;
+    NetGrad g{};
+    g.rows = rows; g.part = gpart; g.csum = cs_part;
+    long p0 = 0, c0 = 0;
     for (int l = 0; l < MLP_LAYERS; ++l) {
-        if ((e = mlp_adam(W32[l], gW[l], mW[l], vW[l], W16[l], wsize(l), lr, ADAM_B1, ADAM_B2, ADAM_EPS, c1, c2, st)) !=
-            hipSuccess)
-            return e;
-        if ((e = mlp_adam(b32[l], gb[l], mb[l], vb[l], nullptr, MLP_N[l], lr, ADAM_B1, ADAM_B2, ADAM_EPS, c1, c2, st)) !=
-            hipSuccess)
-            return e;
+        const int tiles = (MLP_K[l] / 64) * (MLP_N[l] / 64);
+        g.K[l] = MLP_K[l]; g.N[l] = MLP_N[l];
+        g.in[l] = l == 0 ? X : H[l - 1];
+        g.z[l] = l == MLP_LAYERS - 1 ? dY : dZ[l];
+        g.split[l] = choose_split(rows, tiles);
+        g.chunk[l] = rows / g.split[l];
+        g.wg[l] = tiles * g.split[l];
+        g.part0[l] = p0; g.csum0[l] = c0;
+        p0 += long(g.split[l]) * wsize(l);
+        c0 += long(rows / 64) * MLP_N[l];
     }
-    return hipSuccess;
+    if ((e = net_gradients(g, st)) != hipSuccess) return e;
+    NetParams p = params();
+    if (lr > 0.0f) {
+        ++step;
+        p.lr = lr; p.b1 = ADAM_B1; p.b2 = ADAM_B2; p.eps = ADAM_EPS;
+        p.c1 = 1.0f - std::pow(ADAM_B1, float(step));
+        p.c2 = 1.0f - std::pow(ADAM_B2, float(step));
+    }
+    return net_update(p, g, st);
 }
 
 hipError_t Surrogate::network(FeatArgs fa, const int *list, const unsigned *list_n, int rows_max, hipStream_t st) {
@@ -213,11 +186,10 @@ hipError_t Surrogate::fallback(ChemArgs ca, int chem_wg, hipStream_t st) {
 
 Surrogate::~Surrogate() {
     auto f = [](void *p) { if (p) (void)hipFree(p); };
-    for (int l = 0; l < MLP_LAYERS; ++l) {
-        f(W32[l]); f(b32[l]); f(W16[l]); f(mW[l]); f(vW[l]); f(mb[l]); f(vb[l]); f(gW[l]); f(gb[l]);
-    }
+    f(flat);
     for (int l = 0; l < 4; ++l) { f(H[l]); f(Pre[l]); }
-    for (int i = 0; i < 2; ++i) { f(Hping[i]); f(dZ[i]); }
+    for (int i = 0; i < 4; ++i) f(dZ[i]);
+    f(Wfwd); f(Wbwd);
     f(X); f(Yh); f(Yt); f(dY); f(gpart); f(cs_part); f(loss_part); f(d_loss); f(in_range); f(fb_list);
     f(stiff); f(d_stiff_n); f(d_nfb); f(d_norm); f(d_ncf); f(cand_list); f(cand); f(d_ncand);
     if (stream) (void)hipStreamDestroy(stream);
@@ -250,21 +222,25 @@ int fcfd_sur_create(const fcfd_mech *m, fcfd_surrogate **out) {
     auto s = std::make_unique<fcfd_surrogate>();
     s->mech = m;
     HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
+    // parameters, gradients and moments: each one array in the order of fcfd_sur_set_params
+    const size_t np = size_t(fcfd_sur_nparams());
+    HIP_TRY(hipMalloc(&s->flat, 4 * np * 4));
+    HIP_TRY(hipMemset(s->flat, 0, 4 * np * 4));
+    float *at = s->flat;
     for (int l = 0; l < MLP_LAYERS; ++l) {
-        const size_t w = size_t(wsize(l)), b = size_t(MLP_N[l]);
-        HIP_TRY(hipMalloc(&s->W32[l], w * 4)); HIP_TRY(hipMalloc(&s->W16[l], w * 2));
-        HIP_TRY(hipMalloc(&s->mW[l], w * 4)); HIP_TRY(hipMalloc(&s->vW[l], w * 4)); HIP_TRY(hipMalloc(&s->gW[l], w * 4));
-        HIP_TRY(hipMalloc(&s->b32[l], b * 4)); HIP_TRY(hipMalloc(&s->mb[l], b * 4)); HIP_TRY(hipMalloc(&s->vb[l], b * 4));
-        HIP_TRY(hipMalloc(&s->gb[l], b * 4));
-        HIP_TRY(hipMemset(s->W32[l], 0, w * 4)); HIP_TRY(hipMemset(s->W16[l], 0, w * 2));
-        HIP_TRY(hipMemset(s->mW[l], 0, w * 4)); HIP_TRY(hipMemset(s->vW[l], 0, w * 4));
-        HIP_TRY(hipMemset(s->b32[l], 0, b * 4)); HIP_TRY(hipMemset(s->mb[l], 0, b * 4)); HIP_TRY(hipMemset(s->vb[l], 0, b * 4));
+        s->W32[l] = at; s->gW[l] = at + np; s->mW[l] = at + 2 * np; s->vW[l] = at + 3 * np;
+        at += wsize(l);
+        s->b32[l] = at; s->gb[l] = at + np; s->mb[l] = at + 2 * np; s->vb[l] = at + 3 * np;
+        at += MLP_N[l];
     }
-    size_t gp = 0;                       // largest split-K partial set (see choose_split)
+    size_t gp = 0, nw = 0;               // largest split-K partial sets (see choose_split), weights
     for (int l = 0; l < MLP_LAYERS; ++l) {
         const int tiles = (MLP_K[l] / 64) * (MLP_N[l] / 64);
-        gp = std::max(gp, size_t(std::max(1, 256 / tiles)) * size_t(wsize(l)));
+        gp += size_t(std::max(1, 256 / tiles)) * size_t(wsize(l));
+        nw += size_t(wsize(l));
     }
+    HIP_TRY(hipMalloc(&s->Wfwd, nw * 2)); HIP_TRY(hipMalloc(&s->Wbwd, nw * 2));
+    HIP_TRY(hipMemset(s->Wfwd, 0, nw * 2)); HIP_TRY(hipMemset(s->Wbwd, 0, nw * 2));
     HIP_TRY(hipMalloc(&s->gpart, gp * 4));
     HIP_TRY(hipMalloc(&s->d_loss, 4));
     HIP_TRY(hipMalloc(&s->d_nfb, sizeof(unsigned)));
@@ -295,18 +271,10 @@ int fcfd_sur_nparams(void) {
 
 int fcfd_sur_set_params(fcfd_surrogate *s, const float *params) {
     if (!s || !params) { set_error("fcfd_sur_set_params: invalid argument"); return FCFD_E_ARG; }
-    const float *p = params;
-    for (int l = 0; l < MLP_LAYERS; ++l) {
-        HIP_TRY(hipMemcpyAsync(s->W32[l], p, wsize(l) * 4, hipMemcpyHostToDevice, s->stream));
-        p += wsize(l);
-        HIP_TRY(hipMemcpyAsync(s->b32[l], p, MLP_N[l] * 4, hipMemcpyHostToDevice, s->stream));
-        p += MLP_N[l];
-        HIP_TRY(mlp_to_bf16(s->W32[l], s->W16[l], wsize(l), s->stream));
-        HIP_TRY(hipMemsetAsync(s->mW[l], 0, wsize(l) * 4, s->stream));
-        HIP_TRY(hipMemsetAsync(s->vW[l], 0, wsize(l) * 4, s->stream));
-        HIP_TRY(hipMemsetAsync(s->mb[l], 0, MLP_N[l] * 4, s->stream));
-        HIP_TRY(hipMemsetAsync(s->vb[l], 0, MLP_N[l] * 4, s->stream));
-    }
+    const size_t np = size_t(fcfd_sur_nparams());
+    HIP_TRY(hipMemcpyAsync(s->flat, params, np * 4, hipMemcpyHostToDevice, s->stream));
+    HIP_TRY(hipMemsetAsync(s->flat + 2 * np, 0, 2 * np * 4, s->stream));
+    HIP_TRY(net_pack(s->params(), s->stream));
     s->step = 0;
     HIP_TRY(hipStreamSynchronize(s->stream));
     return FCFD_OK;
@@ -314,26 +282,15 @@ int fcfd_sur_set_params(fcfd_surrogate *s, const float *params) {
 
 int fcfd_sur_get_params(fcfd_surrogate *s, float *params) {
     if (!s || !params) { set_error("fcfd_sur_get_params: invalid argument"); return FCFD_E_ARG; }
-    float *p = params;
-    for (int l = 0; l < MLP_LAYERS; ++l) {
-        HIP_TRY(hipMemcpyAsync(p, s->W32[l], wsize(l) * 4, hipMemcpyDeviceToHost, s->stream));
-        p += wsize(l);
-        HIP_TRY(hipMemcpyAsync(p, s->b32[l], MLP_N[l] * 4, hipMemcpyDeviceToHost, s->stream));
-        p += MLP_N[l];
-    }
+    HIP_TRY(hipMemcpyAsync(params, s->flat, size_t(fcfd_sur_nparams()) * 4, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     return FCFD_OK;
 }
 
 int fcfd_sur_get_grads(fcfd_surrogate *s, float *grads) {
     if (!s || !grads) { set_error("fcfd_sur_get_grads: invalid argument"); return FCFD_E_ARG; }
-    float *p = grads;
-    for (int l = 0; l < MLP_LAYERS; ++l) {
-        HIP_TRY(hipMemcpyAsync(p, s->gW[l], wsize(l) * 4, hipMemcpyDeviceToHost, s->stream));
-        p += wsize(l);
-        HIP_TRY(hipMemcpyAsync(p, s->gb[l], MLP_N[l] * 4, hipMemcpyDeviceToHost, s->stream));
-        p += MLP_N[l];
-    }
+    const size_t np = size_t(fcfd_sur_nparams());
+    HIP_TRY(hipMemcpyAsync(grads, s->flat + np, np * 4, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     return FCFD_OK;
 }
@@ -386,7 +343,6 @@ int fcfd_sur_targets(fcfd_surrogate *s, int n, const double *T0, const double *Y
 int fcfd_sur_forward(fcfd_surrogate *s, int rows, const void *X, float *Yh, void *stream) {
     if (!s || rows < 64 || rows % 64 || !X || !Yh) { set_error("fcfd_sur_forward: rows must be a positive multiple of 64"); return FCFD_E_ARG; }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    HIP_TRY(s->reserve(std::min(rows, INFER_CHUNK), false));
     HIP_TRY(s->forward(static_cast<const uint16_t *>(X), rows, Yh, false, st));
     HIP_TRY(hipStreamSynchronize(st));
     return FCFD_OK;
@@ -402,8 +358,7 @@ int fcfd_sur_train_step(fcfd_surrogate *s, const void *X_all, const float *Tg_al
     HIP_TRY(s->reserve(batch, true));
     HIP_TRY(mlp_gather_bf16(static_cast<const uint16_t *>(X_all), s->X, idx, batch, MLP_INP, st));
     HIP_TRY(mlp_gather_f32(Tg_all, s->Yt, idx, batch, MLP_OUTP, st));
-    HIP_TRY(s->backward(batch, st));
-    if (lr > 0.0f) HIP_TRY(s->adam(lr, st));
+    HIP_TRY(s->train(batch, lr, st));
     if (loss) {
         HIP_TRY(hipMemcpyAsync(loss, s->d_loss, 4, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
@@ -452,7 +407,7 @@ int fcfd_bf16_gemm(int M, int N, int K, const void *A, long sam, long sak, const
     GemmArgs g{};
     g.A = static_cast<const uint16_t *>(A); g.B = static_cast<const uint16_t *>(B);
     g.sam = sam; g.sak = sak; g.sbk = sbk; g.sbn = sbn; g.M = M; g.N = N; g.K = K; g.ksplit = ksplit;
-    g.C32 = C; g.ldc = ldc; g.epilogue = EP_STORE;
+    g.C32 = C; g.ldc = ldc;
     hipError_t e = launch_gemm(g, static_cast<hipStream_t>(stream));
     if (e == hipErrorInvalidValue) { set_error("fcfd_bf16_gemm: M, N must be multiples of 64 and K / ksplit a multiple of 16"); return FCFD_E_ARG; }
     HIP_TRY(e);

@@ -57,6 +57,49 @@ struct ApplyArgs {
     double resid_tol, t_tol;
 };
 
+// A pass through the network (mlp_net.hip); rows a multiple of 64.
+struct NetArgs {
+    const uint16_t *x;           // [rows][64]: features (forward) or the output's gradient (backward)
+    const uint16_t *w;           // packed weights (NetParams::fwd or bwd)
+    const float *bias[MLP_LAYERS];
+    int rows;
+    int wide;                    // 1: x and out are aligned to 16 bytes
+    float *out;                  // forward: [rows][64]
+    // hidden layers, in the order the pass meets them: training's forward writes pre-activations P and
+    // activations H, backward reads P and writes the gradients of the pre-activations to H
+    uint16_t *H[4];
+    float *P[4];
+    // inference, optional: device count of live rows and, with it, per-row flags; 64-row tiles past the
+    // count or without a flag set are not evaluated, their output rows left as they were
+    const unsigned *m_dev;
+    const int *row_live;
+};
+hipError_t net_forward(const NetArgs &a, bool training, hipStream_t st);
+hipError_t net_backward(const NetArgs &a, hipStream_t st);
+
+// Weight and bias gradients: inputs and output gradients of every layer, the split of the rows and the
+// partial sums' places.
+struct NetGrad {
+    int rows;
+    int K[MLP_LAYERS], N[MLP_LAYERS];
+    const uint16_t *in[MLP_LAYERS], *z[MLP_LAYERS];
+    int split[MLP_LAYERS], chunk[MLP_LAYERS], wg[MLP_LAYERS];      // slices, rows each, workgroups
+    float *part, *csum;
+    long part0[MLP_LAYERS], csum0[MLP_LAYERS];
+};
+hipError_t net_gradients(const NetGrad &g, hipStream_t st);
+
+struct NetParams {
+    int K[MLP_LAYERS], N[MLP_LAYERS];
+    float *W[MLP_LAYERS], *b[MLP_LAYERS], *gW[MLP_LAYERS], *gb[MLP_LAYERS];
+    float *mW[MLP_LAYERS], *vW[MLP_LAYERS], *mb[MLP_LAYERS], *vb[MLP_LAYERS];
+    uint16_t *fwd, *bwd;         // packed BF16 weights
+    int fwd0[MLP_LAYERS], bwd0[MLP_LAYERS];
+    float lr, b1, b2, eps, c1, c2;
+};
+hipError_t net_pack(const NetParams &p, hipStream_t st);
+hipError_t net_update(const NetParams &p, const NetGrad &g, hipStream_t st);
+
 hipError_t mlp_features(const FeatArgs &f, int rows, hipStream_t st);
 hipError_t mlp_targets(const SurrogateNorm *nm, int kk, int n, int npad, const double *T0, const double *Y0,
                        const double *T1, const double *Y1, float *Tg, hipStream_t st);
@@ -64,11 +107,6 @@ hipError_t mlp_gather_bf16(const uint16_t *src, uint16_t *dst, const int *idx, i
 hipError_t mlp_gather_f32(const float *src, float *dst, const int *idx, int rows, int w, hipStream_t st);
 hipError_t mlp_mse(const float *Yh, const float *Yt, uint16_t *dY, int rows, float *partial, float *loss,
                    hipStream_t st);
-hipError_t mlp_reduce_splits(const float *parts, float *out, int nsplit, long len, hipStream_t st);
-hipError_t mlp_colsum(const uint16_t *D, float *partial, float *out, int rows, int cols, hipStream_t st);
-hipError_t mlp_adam(float *w, const float *g, float *m, float *v, uint16_t *w16, long n, float lr, float b1, float b2,
-                    float eps, float c1, float c2, hipStream_t st);
-hipError_t mlp_to_bf16(const float *w, uint16_t *w16, long n, hipStream_t st);
 hipError_t mlp_zero_u32(unsigned *p, hipStream_t st);
 hipError_t mlp_apply(const ApplyArgs &a, int nsp, hipStream_t st);
 
