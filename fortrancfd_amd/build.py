@@ -26,9 +26,9 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "-ffp-contract=off", "-Wall",
           f"-I{os.path.join(REPO, 'include')}", f"-I{CSRC}"]
 HIP_FLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-munsafe-fp-atomics"]
-# Per source: chem_coop.hip's command loop keeps what it needs in registers only while the compiler does
-# not move every coefficient of its exponentials and logarithms in front of the loop.
-EXTRA_FLAGS = {"chem_coop.hip": ["-mllvm", "-disable-machine-licm"]}
+# Per source: the rate kernels keep what they need in registers only while the compiler does not move
+# every coefficient of their exponentials and logarithms in front of their loops.
+EXTRA_FLAGS = {src: ["-mllvm", "-disable-machine-licm"] for src in ("chem_coop.hip", "chem_lane.hip")}
 
 
 def build(verbose: bool = False) -> str:

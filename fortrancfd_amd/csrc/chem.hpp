@@ -5,8 +5,9 @@
 
 namespace fcfd {
 
-constexpr int LANE_NW = 8;       // waves per workgroup of the lane-per-cell kernels
-constexpr int LANE_CHUNK = 32;   // reaction rows per chunk of their scatter (four per wave)
+constexpr int LANE_NW = 8;       // waves of a lane-per-cell workgroup that share the species
+constexpr int LANE_RW = 16;      // waves of it that share the reactions
+constexpr int LANE_CHUNK = 7 * LANE_RW;   // reaction rows between two barriers (seven per wave)
 constexpr int LANE_NC = 64;      // cells per workgroup of the lane-per-cell kernels
 
 // A row of the branch-free range (nplain0 .. ii-1) as the lane-per-cell kernels read it, with one
@@ -16,7 +17,7 @@ constexpr int LANE_NC = 64;      // cells per workgroup of the lane-per-cell ker
 struct LanePlain {
     double A, B, E;
     double nud[6];
-    unsigned short off[6];
+    int off[6];
     int bits;                    // LP_* fields
 };
 constexpr int LP_NR = 0;         // bits 0-1: reactant slots (1-3)
@@ -27,11 +28,15 @@ constexpr int LP_NUS = 6;        // bits 6-8: coefficient sum + 3
 constexpr int LP_POW = 1 << 9;   // some slot has |coefficient| > 1
 constexpr int LP_PW = 10;        // bits 10-21: |coefficient| of slot n in bits 10 + 2n .. 11 + 2n
 constexpr int LP_DEAD = 1 << 22; // coefficient of slot 0 is 0: no rate
-// A scatter entry of the lane-per-cell kernels: W[k] += Q[r] * nu with the byte offsets of row k of
-// the production-rate block and row r of the chunk's rate block.
+// The lane-per-cell kernels' sums: a segment is one species' terms of a chunk, n entries from e0 on, added to
+// the production rate at byte offset off; an entry is a rate's byte offset in the chunk's block and the
+// coefficient.
+struct LaneSeg {
+    int off, e0, n;
+};
 struct LaneEnt {
-    int offW, offQ;
     double nu;
+    int off, pad;
 };
 
 // ---- tables of the integrator that gives a cell eight waves (chem_coop.hip) ----
@@ -68,12 +73,14 @@ struct DevKin {
     int ifop[MAXR], kfal[MAXR];         // fall-off form (1 Lindemann, 2 SRI, 3/4 Troe), [M] species
     double fpar[MAXR][8];
     int orig[MAXR];                     // the mechanism's (0-based) index of each device row
-    // scatter lists of the lane-per-cell kernels (chem_lane.hip): rows are taken in chunks of
-    // LANE_CHUNK; within chunk c, wave w adds the entries lane_ent[lane_ent0[c * LANE_NW + w] ..
-    // lane_ent0[c * LANE_NW + w + 1]) to the production rates of the species it owns (k mod LANE_NW
-    // = w), in row then slot order.
-    int lane_ent0[(MAXR + LANE_CHUNK - 1) / LANE_CHUNK * LANE_NW + 1];
+    // lists of the lane-per-cell kernels (chem_lane.hip): rows are taken in chunks of LANE_CHUNK; after
+    // chunk c, wave w sums the segments lane_seg[lane_seg0[c * LANE_RW + w] .. lane_seg0[c * LANE_RW + w +
+    // 1]), each in row then slot order.  The species of a chunk go to the waves by their entries, most
+    // first.
+    int lane_seg0[(MAXR + LANE_CHUNK - 1) / LANE_CHUNK * LANE_RW + 1];
+    LaneSeg lane_seg[(MAXR + LANE_CHUNK - 1) / LANE_CHUNK * 64];
     LaneEnt lane_ent[MAXR * 6];
+    int usual;                          // 1: the constants that are divided by T are 0 or in 2^-700 .. 2^60
     LanePlain lane_plain[MAXR];         // rows nplain0 .. ii-1 (other entries unused)
     // Packed rows of the eight-wave integrator: [0] species of slots 0-3, a byte each (COOP_EMPTY: none);
     // [1] those of slots 4 and 5; [2] CR_* and the coefficients as four-bit two's complement in bits

@@ -8,45 +8,152 @@
 // the order of the species sums differs.  k_chem_retry runs the integrator's next explicit attempt
 // (two half steps) the same way over a long work list, before the SDIRK kernel sees it.
 //
-// Mapping: a workgroup of NW = 8 waves owns NC = 64 cells (lane l of every wave is cell l; with
+// Mapping: a workgroup of RW = 16 waves owns NC = 64 cells (lane l of every wave is cell l; with
 // NC < 64, lanes NC..63 would repeat cell NC - 1 and store nothing).  Concentrations and S/R - H/RT of
 // the cells live in LDS as species-major [k][NC] blocks.  The reactions are taken in chunks of
-// CH = 32 rows: each wave evaluates four rows of a chunk for all cells and puts their rates of
-// progress in LDS; after a barrier every wave adds the chunk's contributions to the species it owns
-// (k mod NW = wave) from a precomputed list, in row order, into one shared production-rate block
-// whose rows no two waves write.  Each species' production rate is therefore one sequential sum over
-// the rows, independent of the wave count.  Species-wise work (thermo, state update, norms) is split
-// over the waves by k mod NW; cell-wise scalars (T, sums) are combined through LDS in wave order.
-// The LDS footprint (~101 KB) holds one workgroup per compute unit: two waves per SIMD, and every
-// lane a cell, so 65,536 cells make exactly four rounds of 1024 workgroups on 256 CUs.  Reaction
-// tables are read with a wave-uniform row index (scalar loads).
+// CH = 112 rows: the waves draw rows from a counter, evaluate each for all cells and put its rates of
+// progress in LDS; after a barrier every wave adds the chunk's contributions to the species it was given
+// (LaneSeg: by their number of terms), in row order, into one shared production-rate block.  Each
+// species' production rate is therefore one sequential sum over the rows, independent of which wave does
+// what.  Species-wise work (thermo, state update, norms) is split over the first NW = 8 waves by k mod
+// NW; cell-wise scalars (T, sums) are combined through LDS in wave order, by every wave.
+//
+// Bound: the issue of one SIMD's four waves.  A plain row takes some 120 vector operations (two
+// exponentials, a division), a fall-off row 500; 325 rows are 62k cycles of a SIMD, of which a right-hand
+// side took 100k, and 35k more go to the species' terms and the sums.  LDS (143 KB) holds one workgroup
+// per compute unit; 128 registers a lane allow its 16 waves.  65,536 cells (four rounds of 256
+// workgroups): 682 us a launch, 510 cells: 181 us.  Eight waves with 32-row chunks, one fixed row in
+// eight each, and table reads that went through the vector cache at each branch took 1,098 and 334 us.
 #include <algorithm>
 
 #include "chem.hpp"
 #include "chem_device.hpp"
 #include "fcfd_device.hpp"
+#include "rate_math.hpp"
 
 namespace fcfd {
 
 namespace {
 
-constexpr int NW = LANE_NW;    // waves per workgroup
+constexpr int NW = LANE_NW;    // waves that own species
+constexpr int RW = LANE_RW;    // waves per workgroup, each with rows of a chunk
 constexpr int NC = LANE_NC;    // cells per workgroup
-constexpr int CH = LANE_CHUNK; // reaction rows per chunk, CH / NW per wave
-constexpr int RB = CH / NW;
+constexpr int CH = LANE_CHUNK; // reaction rows per chunk
 
 template <int NSP>
 struct LaneShared {
     double C[NSP * NC];        // concentrations, mol/cm^3
     double G[NSP * NC];        // S/R - H/RT
-    double W[NSP * NC];        // production rates; row k is written by wave k mod NW only
+    double W[NSP * NC];        // production rates
     double Q[CH * NC];         // rates of progress (forward minus reverse) of the current chunk; outside
                                // the reaction loop, the per-wave values of cross-wave sums
+    int next[2];               // rows of a chunk handed out, by the chunk's parity
     double PF[7 * NC];         // pfac**m for m = -3 .. 3 (row m + 3), the equilibrium constants' factor
 };
 
-// reaction_plain (chem_device.hpp) for a row the whole wave evaluates (wave-uniform row index), as
-// forward minus reverse rate of progress: the same operations, with the slot counts, coefficient
+// The tables through the constant address space: reads at a wave-uniform index are scalar loads wherever
+// they stand (behind a barrier or an LDS store they would otherwise go through the vector caches, one
+// after the other as a row's branches ask for them).
+using CKin = const __attribute__((address_space(4))) DevKin;
+using CLanePlain = const __attribute__((address_space(4))) LanePlain;
+
+// Both coefficient sets as scalars, the range selected per lane.  (Opaque: a compiler that sees the loads
+// selects their address instead, which makes each a memory access per lane.)
+__device__ __forceinline__ Nasa nasa(CThermo *m, int k, double T) {
+    const bool up = T > m->tmid[k];
+    auto pick = [&](int n) {
+        double lo = m->alo[k][n], hi = m->ahi[k][n];
+        asm("" : "+s"(lo));
+        asm("" : "+s"(hi));
+        return up ? hi : lo;
+    };
+    return Nasa{pick(0), pick(1), pick(2), pick(3), pick(4), pick(5), pick(6)};
+}
+
+// a / T for a table constant
+__device__ __forceinline__ double over(double a, const Temp &t, bool usual) {
+    double q = over(a, t);
+    if (__builtin_expect(!usual, 0)) q = a / t.T;       // (the same in all lanes)
+    return q;
+}
+
+// reaction() (chem_device.hpp) for a row the whole wave evaluates, as forward minus reverse rate of
+// progress: the same operations, with the exponentials and logarithms of rate_math.hpp and T's
+// reciprocal.
+__device__ __forceinline__ double lane_row_q(CKin *K, CSeries *ks, int i, const Temp &tp, bool usual,
+                                             double pfac, double ctot, const double *__restrict__ c,
+                                             const double *__restrict__ smh) {
+    auto nu = &K->nu[i][0], nk = &K->nk[i][0];
+    if (nu[0] == 0) return 0.0;
+    double kf = K->A[i];
+    if (!K->arr0[i]) kf = kf * exp_rate(ks, K->B[i] * tp.logT - over(K->E[i], tp, usual));
+    double kr = 0.0;
+    if (K->rev[i]) {
+        double s = 0.0;
+        for (int n = 0; n < 6; ++n) {
+            const int k = nk[n];
+            if (k >= 0) s = s + (double)nu[n] * smh[k * NC];
+        }
+        double eqk = s != 0.0 ? exp_rate(ks, fmin(s, K->exparg)) : 1.0;
+        eqk = eqk * ipow(pfac, K->nus[i]);
+        kr = kf / fmax(eqk, K->small);
+    }
+    double ctb = 1.0;
+    const int t = K->tb[i];
+    if (t >= 0) {
+        ctb = ctot;
+        const int nl = K->ntbs[t];
+        for (int l = 0; l < nl; ++l) {
+            const int tk = K->tbk[t][l];
+            ctb = ctb + (K->tba[t][l] - 1.0) * c[(tk >= 0 ? tk : 0) * NC];
+        }
+    }
+    const int f = K->fo[i];
+    if (f >= 0) {
+        auto fp = &K->fpar[f][0];
+        const double rklow = fp[0] * exp_rate(ks, fp[1] * tp.logT - over(fp[2], tp, usual));
+        double pr;
+        if (K->kfal[f] < 0) { pr = rklow * ctb / kf; ctb = 1.0; }
+        else pr = rklow * c[K->kfal[f] * NC] / kf;
+        double pcor = pr / (1.0 + pr);
+        if (K->ifop[f] > 1) {
+            const double prlog = log10_rate(ks, fmax(pr, K->small));
+            double fc;
+            if (K->ifop[f] == 2) {
+                const double xp = 1.0 / (1.0 + prlog * prlog);
+                fc = fm_pow(fp[3] * fm_exp(-fp[4] / tp.T) + fm_exp(-tp.T / fp[5]), xp) * fp[6] * fm_pow(tp.T, fp[7]);
+            } else {
+                double fcent = (1.0 - fp[3]) * exp_rate(ks, -tp.T / fp[4]) + fp[3] * exp_rate(ks, -tp.T / fp[5]);
+                if (K->ifop[f] == 4) fcent = fcent + exp_rate(ks, -over(fp[6], tp, usual));
+                const double fclog = log10_rate(ks, fmax(fcent, K->small));
+                // single-precision literals of cklib.f:6915-6917
+                const double xn = 0.75 - (double)1.27f * fclog;
+                const double cprlog = prlog - ((double)0.4f + (double)0.67f * fclog);
+                const double q = cprlog / (xn - (double)0.14f * cprlog);
+                fc = exp10_rate(ks, fclog / (1.0 + q * q));
+            }
+            pcor = fc * pcor;
+        }
+        kf = kf * pcor;
+        kr = kr * pcor;
+    }
+    kf = kf * ctb * 1.0;
+    kr = kr * ctb * 1.0;
+    double qf = kf * ipow(c[nk[0] * NC], abs(nu[0]));
+    double qr = kr * ipow(c[nk[3] * NC], nu[3]);
+    if (nk[1] >= 0) {
+        qf = qf * ipow(c[nk[1] * NC], abs(nu[1]));
+        if (nk[2] >= 0) qf = qf * ipow(c[nk[2] * NC], abs(nu[2]));
+    }
+    if (nk[4] >= 0) {
+        qr = qr * ipow(c[nk[4] * NC], nu[4]);
+        if (nk[5] >= 0) qr = qr * ipow(c[nk[5] * NC], nu[5]);
+    }
+    return qf - qr;
+}
+
+// reaction_plain (chem_device.hpp) for a row the whole wave evaluates, as forward minus reverse rate of
+// progress: the same operations, with the slot counts, coefficient
 // powers and flags of K->lane_plain taken as scalar branches instead of selects, the species rows
 // read at byte offsets from this lane's column of the C and G blocks, and pfac**nus from the lane's
 // PF column.  Multiplications by exactly 1.0 that reaction_plain makes for empty slots are skipped
@@ -57,27 +164,43 @@ __device__ __forceinline__ double ipow_u(double x, int m) {      // ipow3 for a 
     return m == 2 ? x2 : x * x2;
 }
 
-__device__ __forceinline__ double lane_plain_q(const LanePlain *__restrict__ L, double T, double alogt,
-                                               double small, double exparg, const char *Cb, const char *Gb,
+__device__ __forceinline__ double lane_plain_q(CLanePlain *L, CSeries *ks, const Temp &tp, bool usual,
+                                               double small, double exparg, const char *Cb, int dG,
                                                const double *Pf) {
+    // the whole record at once: one wait instead of one at each branch
     const int bits = L->bits;
+    const double A = L->A, B = L->B, E = L->E;
+    const double nud[6] = {L->nud[0], L->nud[1], L->nud[2], L->nud[3], L->nud[4], L->nud[5]};
+    const int off[6] = {L->off[0], L->off[1], L->off[2], L->off[3], L->off[4], L->off[5]};
     if (bits & LP_DEAD) return 0.0;
     const int nr = (bits >> LP_NR) & 3, np = (bits >> LP_NP) & 3;
-    auto C = [&](int n) { return *reinterpret_cast<const double *>(Cb + L->off[n]); };
-    auto G = [&](int n) { return *reinterpret_cast<const double *>(Gb + L->off[n]); };
-    double kf = L->A;
-    if (!(bits & LP_ARR0)) kf = kf * fm_exp(L->B * alogt - L->E / T);
+    // concentrations and S/R - H/RT of the filled slots (G follows C at a constant distance)
+    double c[6] = {}, g[6] = {};
+    auto read = [&](int n) {
+        const char *at = Cb + off[n];
+        c[n] = *reinterpret_cast<const double *>(at);
+        g[n] = *reinterpret_cast<const double *>(at + dG);
+    };
+    read(0);
+    if (nr >= 2) read(1);
+    if (nr >= 3) read(2);
+    if (np >= 1) read(3);
+    if (np >= 2) read(4);
+    if (np >= 3) read(5);
+    auto C = [&](int n) { return c[n]; };
+    double kf = A;
+    if (!(bits & LP_ARR0)) kf = kf * exp_near(ks, B * tp.logT - over(E, tp, usual));
     double kr = 0.0;
     if (bits & LP_REV) {
         // reaction_plain starts from 0.0 + t0; the two differ at most in the sign of a zero sum,
         // which the test s != 0 and exp(+-0) = 1 do not see
-        double s = L->nud[0] * G(0);
-        if (nr >= 2) s = s + L->nud[1] * G(1);
-        if (nr >= 3) s = s + L->nud[2] * G(2);
-        if (np >= 1) s = s + L->nud[3] * G(3);
-        if (np >= 2) s = s + L->nud[4] * G(4);
-        if (np >= 3) s = s + L->nud[5] * G(5);
-        double eqk = s != 0.0 ? fm_exp(fmin(s, exparg)) : 1.0;
+        double s = nud[0] * g[0];
+        if (nr >= 2) s = s + nud[1] * g[1];
+        if (nr >= 3) s = s + nud[2] * g[2];
+        if (np >= 1) s = s + nud[3] * g[3];
+        if (np >= 2) s = s + nud[4] * g[4];
+        if (np >= 3) s = s + nud[5] * g[5];
+        double eqk = exp_near(ks, fmin(s, exparg));      // (1 for s = 0)
         eqk = eqk * Pf[((bits >> LP_NUS) & 7) * NC];
         kr = kf / fmax(eqk, small);
     }
@@ -101,14 +224,15 @@ __device__ __forceinline__ double lane_plain_q(const LanePlain *__restrict__ L, 
     return qf - qr;
 }
 
-// Species slots of wave w: k = w + NW * j.
+// Species slots of wave w < NW: k = w + NW * j; the other waves have none (species_base: past the last).
+__device__ __forceinline__ int species_base(int w) { return w < NW ? w : 1 << 20; }
 template <int NSP>
 constexpr int slots() { return (NSP + NW - 1) / NW; }
 
 // Sum over the NW waves of one value per cell, in wave order, through a block of NW * NC doubles
 // (the start of the rate block Q, free outside the reaction loop).
 __device__ __forceinline__ double sum_waves(double *slot, int w, int cl, double v) {
-    slot[w * NC + cl] = v;
+    if (w < NW) slot[w * NC + cl] = v;
     __syncthreads();
     double s = slot[cl];
 #pragma unroll
@@ -120,8 +244,10 @@ __device__ __forceinline__ double sum_waves(double *slot, int w, int cl, double 
 // The same for two values at once through a block of 2 * NW * NC doubles (the rate block Q, free
 // outside the reaction loop): one pair of barriers instead of two.
 __device__ __forceinline__ void sum_waves2(double *pair, int w, int cl, double va, double vb, double &ra, double &rb) {
-    pair[w * NC + cl] = va;
-    pair[(NW + w) * NC + cl] = vb;
+    if (w < NW) {
+        pair[w * NC + cl] = va;
+        pair[(NW + w) * NC + cl] = vb;
+    }
     __syncthreads();
     const double *q = pair + NW * NC;
     ra = pair[cl];
@@ -137,7 +263,7 @@ __device__ __forceinline__ void sum_waves2(double *pair, int w, int cl, double v
 // f = dy/dt at (y + s d, T) for this wave's species slots (f[j] of species w + NW*j) and fT for
 // all waves (SHIFT = false: at y).  rho in g/cm^3.  cl: this lane's LDS column.
 template <int NSP, bool SHIFT>
-__device__ __forceinline__ void rhs_lane(const DevThermo *__restrict__ th, const DevKin *__restrict__ K, LaneShared<NSP> &sh,
+__device__ __forceinline__ void rhs_lane(CThermo *th, CKin *K, LaneShared<NSP> &sh,
                          int w, int cl, double rho, const double (&y)[slots<NSP>()],
                          const double (&d)[slots<NSP>()], double s, double T, double (&f)[slots<NSP>()],
                          double &fT) {
@@ -145,10 +271,16 @@ __device__ __forceinline__ void rhs_lane(const DevThermo *__restrict__ th, const
     const TPow p = tpow(T, th->ru);
     double uk[NS];
     double ctot_w = 0.0, cvm_w = 0.0;
-    const double lnT = fm_log(T);
+    CSeries *ks = get_series();
+    Temp tp = temperature(ks, T);
+    // beyond any temperature of a state that can be accepted: NaN rates, the cell goes on to the integrator.
+    // (Arguments of exp_near stay below 2^30.)
+    tp.logT = T >= 0x1p-7 && T <= 0x1p27 ? tp.logT : __builtin_nan("");
+    const double lnT = tp.logT;
+    const bool usual = K->usual != 0;
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        const int k = w + NW * j;
+        const int k = species_base(w) + NW * j;
         uk[j] = 0.0;
         if (k < NSP) {
             const double yj = SHIFT ? y[j] + s * d[j] : y[j];
@@ -182,53 +314,51 @@ __device__ __forceinline__ void rhs_lane(const DevThermo *__restrict__ th, const
     double ctot, cvm;
     sum_waves2(sh.Q, w, cl, ctot_w, cvm_w, ctot, cvm);     // its barrier also publishes C, G and PF
     const double *Cp = sh.C + cl, *Gp = sh.G + cl;
-    const char *Cb = reinterpret_cast<const char *>(Cp), *Gb = reinterpret_cast<const char *>(Gp);
+    const char *Cb = reinterpret_cast<const char *>(Cp);
+    const int dG = int(reinterpret_cast<const char *>(sh.G) - reinterpret_cast<const char *>(sh.C));
     const double *Pf = sh.PF + cl;
     double *Wp = sh.W + cl;
     char *Wb = reinterpret_cast<char *>(Wp);
     const double *Qp = sh.Q + cl;
     const char *Qb = reinterpret_cast<const char *>(Qp);
-    for (int c0 = 0, chunk = 0; c0 < K->ii; c0 += CH, ++chunk) {
-        // this wave's RB rows of the chunk: independent rate chains, so their table loads, LDS
-        // reads and transcendental evaluations overlap
-        const int i0 = c0 + w;
-        double q[RB];
-        if (i0 >= K->nplain0) {
-#pragma unroll
-            for (int u = 0; u < RB; ++u) {
-                const int i = i0 + NW * u;
-                q[u] = i < K->ii ? lane_plain_q(&K->lane_plain[i], T, lnT, K->small, K->exparg, Cb, Gb, Pf) : 0.0;
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < RB; ++u) {
-                const int i = i0 + NW * u;
-                q[u] = 0.0;
-                if (i < K->ii) {
-                    const Rop r = reaction<NC>(K, i, T, lnT, pfac, ctot, Cp, Gp);
-                    q[u] = r.qf - r.qr;
-                }
-            }
+    const int ii = K->ii, np0 = K->nplain0;
+    const double small = K->small, exparg = K->exparg;
+    for (int c0 = 0, chunk = 0; c0 < ii; c0 += CH, ++chunk) {
+        // the chunk's rows, handed out one by one: the waves of a SIMD do not run at the same speed (the
+        // oldest goes first), and the fall-off rows, the first ones, take five times as long
+        const int n = min(CH, ii - c0);
+        for (;;) {
+            int r = 0;
+            if ((threadIdx.x & 63) == 0) r = atomicAdd(&sh.next[chunk & 1], 1);
+            r = __builtin_amdgcn_readfirstlane(r);
+            if (r >= n) break;
+            const int i = c0 + r;
+            const double q = i >= np0 ? lane_plain_q(&K->lane_plain[i], ks, tp, usual, small, exparg, Cb, dG, Pf)
+                                      : lane_row_q(K, ks, i, tp, usual, pfac, ctot, Cp, Gp);
+            sh.Q[r * NC + cl] = q;
         }
-#pragma unroll
-        for (int u = 0; u < RB; ++u) sh.Q[(w + NW * u) * NC + cl] = q[u];
         __syncthreads();
-        // the chunk's contributions to this wave's species, in row then slot order
-        const int e1 = K->lane_ent0[chunk * NW + w + 1];
-        for (int e = K->lane_ent0[chunk * NW + w]; e < e1; ++e) {
-            const LaneEnt &en = K->lane_ent[e];
-            double *wk = reinterpret_cast<double *>(Wb + en.offW);
-            *wk = *wk + *reinterpret_cast<const double *>(Qb + en.offQ) * en.nu;
+        if (threadIdx.x == 0) sh.next[chunk & 1] = 0;       // (used again two chunks on)
+        // the chunk's contributions, species by species
+        const int s1 = K->lane_seg0[chunk * RW + w + 1];
+        for (int sg = K->lane_seg0[chunk * RW + w]; sg < s1; ++sg) {
+            const int goff = K->lane_seg[sg].off, e0 = K->lane_seg[sg].e0, n = K->lane_seg[sg].n;
+            double *wk = reinterpret_cast<double *>(Wb + goff);
+            double s = *wk;
+#pragma unroll 4
+            for (int e = e0; e < e0 + n; ++e)
+                s = s + *reinterpret_cast<const double *>(Qb + K->lane_ent[e].off) * K->lane_ent[e].nu;
+            *wk = s;
         }
         __syncthreads();                   // Q is rewritten by the next chunk
     }
     double su_w = 0.0;
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        const int k = w + NW * j;
+        const int k = species_base(w) + NW * j;
         f[j] = 0.0;
         if (k < NSP) {
-            const double wd = Wp[k * NC];  // a row this wave wrote
+            const double wd = Wp[k * NC];
             f[j] = wd * th->wt[k] / rho;
             su_w = su_w + uk[j] * wd;
         }
@@ -239,14 +369,14 @@ __device__ __forceinline__ void rhs_lane(const DevThermo *__restrict__ th, const
 
 // Mixture e = sum Y u / W and cv (erg/g) over all species at T for this cell.
 template <int NSP>
-__device__ __forceinline__ void energy_lane(const DevThermo *__restrict__ th, double *pair, int w, int lane,
+__device__ __forceinline__ void energy_lane(CThermo *th, double *pair, int w, int lane,
                             const double (&y)[slots<NSP>()], double T, double &e, double &cv) {
     constexpr int NS = slots<NSP>();
     const TPow p = tpow(T, th->ru);
     double eu = 0.0, ec = 0.0;
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        const int k = w + NW * j;
+        const int k = species_base(w) + NW * j;
         if (k < NSP) {
             const Nasa a = nasa(th, k, T);
             eu = eu + y[j] * (h_mol(a, p) - p.rut) / th->wt[k];
@@ -263,7 +393,7 @@ __device__ __forceinline__ void adjust_lane(double *slot, int w, int lane, doubl
     double s = 0.0;
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        y[j] = (w + NW * j < NSP) ? fmax(y[j], 0.0) : 0.0;
+        y[j] = (species_base(w) + NW * j < NSP) ? fmax(y[j], 0.0) : 0.0;
         s = s + y[j];
     }
     const double tot = sum_waves(slot, w, lane, s);
@@ -272,7 +402,7 @@ __device__ __forceinline__ void adjust_lane(double *slot, int w, int lane, doubl
 }
 
 template <int NSP>
-__global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
+__global__ void __launch_bounds__(64 * RW) k_chem_screen(ChemArgs a) {
     constexpr int NS = slots<NSP>();
     __shared__ LaneShared<NSP> sh;
     // the wave index is uniform across the wave; saying so turns every table read indexed by it
@@ -280,8 +410,8 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
     // reaction kind into a scalar branch
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = min(int(threadIdx.x & 63), NC - 1);   // the LDS column (lanes >= NC repeat NC - 1)
-    const DevThermo *__restrict__ th = a.thermo;
-    const DevKin *__restrict__ K = a.kin;
+    CThermo *th = constant(a.thermo);
+    CKin *K = (CKin *)a.kin;
     const int cell0 = int(xcd_block()) * NC;   // neighbouring cell ranges share their XCD's L2
     const int cell = cell0 + lane;
     // every lane of a column takes the column's decisions (lanes >= NC share column NC - 1 and must
@@ -290,6 +420,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
     const bool owner = live && int(threadIdx.x & 63) < NC;
     const int c = live ? cell : cell0;          // columns past the end shadow a live cell
     double *slot = sh.Q;
+    if (threadIdx.x < 2) sh.next[threadIdx.x] = 0;      // (barriers before the first rows)
 
     long col = 0;
     double rho_si, dt, T0;
@@ -302,7 +433,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
         dt = a.dt_dev ? *a.dt_dev : a.dt;
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int k = w + NW * j;
+            const int k = species_base(w) + NW * j;
             y[j] = k < NSP ? a.qf[(3 + k) * a.P + col] : 0.0;
         }
         adjust_lane<NSP>(slot, w, lane, y);
@@ -312,7 +443,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
         T0 = a.b_T[c];
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int k = w + NW * j;
+            const int k = species_base(w) + NW * j;
             y[j] = k < NSP ? a.b_y[long(k) * a.ncells + c] : 0.0;
         }
     }
@@ -335,7 +466,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
     double err_w = 0.0;
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        if (w + NW * j < NSP) {
+        if (species_base(w) + NW * j < NSP) {
             const double wt = 1.0 / (a.atol + a.rtol * fabs(y[j]));
             const double t = ((dt * 0.5) * (f1[j] - f0[j])) * wt;
             err_w = err_w + t * t;
@@ -351,7 +482,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
     if (!ok && owner && a.f0) {   // f at the start state, for the retry of a long list
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int k = w + NW * j;
+            const int k = species_base(w) + NW * j;
             if (k < NSP) a.f0[long(k) * a.ncells + cell] = f0[j];
         }
         if (w == 0) a.f0[long(NSP) * a.ncells + cell] = f0T;
@@ -394,7 +525,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
         double s1 = 0.0, s2 = 0.0;
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int k = w + NW * j;
+            const int k = species_base(w) + NW * j;
             if (k < NSP) {
                 const double y_in = a.layout == 0 ? a.qf[(3 + k) * a.P + col] : a.b_y[long(k) * a.ncells + c];
                 s1 = s1 + rho * th->h298[k] * (y[j] - y_in) / dt;
@@ -407,7 +538,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
     if (a.layout == 0) {
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int k = w + NW * j;
+            const int k = species_base(w) + NW * j;
             if (k < NSP) a.qf[(3 + k) * a.P + col] = y[j];
         }
         if (w == 0) {
@@ -420,7 +551,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
     } else {
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int k = w + NW * j;
+            const int k = species_base(w) + NW * j;
             if (k < NSP) a.b_y[long(k) * a.ncells + cell] = y[j];
         }
         if (w == 0) a.b_T[cell] = T;
@@ -442,20 +573,20 @@ __global__ void __launch_bounds__(64 * NW) k_chem_screen(ChemArgs a) {
 // a.stiff unchanged with *a.retry_done = 0: the integrator then runs it eight waves per cell and
 // retries each cell itself.  Domain layout only.
 template <int NSP>
-__global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
+__global__ void __launch_bounds__(64 * RW) k_chem_retry(ChemArgs a) {
     constexpr int NS = slots<NSP>();
     __shared__ LaneShared<NSP> sh;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = min(int(threadIdx.x & 63), NC - 1);   // the LDS column (lanes >= NC repeat NC - 1)
-    const DevThermo *__restrict__ th = a.thermo;
-    const DevKin *__restrict__ K = a.kin;
+    CThermo *th = constant(a.thermo);
+    CKin *K = (CKin *)a.kin;
     const int n = int(*a.list_n);
     if (coop_list(a, n)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             *a.retry_done = 0;
             *a.stiff_n = unsigned(n);
         }
-        for (int i = int(blockIdx.x) * (64 * NW) + int(threadIdx.x); i < n; i += int(gridDim.x) * (64 * NW)) a.stiff[i] = a.list[i];
+        for (int i = int(blockIdx.x) * (64 * RW) + int(threadIdx.x); i < n; i += int(gridDim.x) * (64 * RW)) a.stiff[i] = a.list[i];
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.retry_done = 1;
@@ -468,6 +599,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
     const bool owner = live && int(threadIdx.x & 63) < NC;
     const int cell = a.list[live ? item : item0];   // columns past the end shadow a live cell
     double *slot = sh.Q;
+    if (threadIdx.x < 2) sh.next[threadIdx.x] = 0;      // (barriers before the first rows)
 
     const int b = cell / a.ncell, i = cell % a.ncell;
     const long col = long(b) * a.S + a.lv + i;
@@ -477,7 +609,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
     double y[NS];
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        const int k = w + NW * j;
+        const int k = species_base(w) + NW * j;
         y[j] = k < NSP ? a.qf[(3 + k) * a.P + col] : 0.0;
     }
     adjust_lane<NSP>(slot, w, lane, y);
@@ -500,7 +632,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
         if (sub == 0 && a.f0) {   // f at the start state, stored by the screen
 #pragma unroll
             for (int j = 0; j < NS; ++j) {
-                const int k = w + NW * j;
+                const int k = species_base(w) + NW * j;
                 fa[j] = k < NSP ? a.f0[long(k) * a.ncells + cell] : 0.0;
             }
             faT = a.f0[long(NSP) * a.ncells + cell];
@@ -511,7 +643,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
         double err_w = 0.0;
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            if (w + NW * j < NSP) {
+            if (species_base(w) + NW * j < NSP) {
                 const double wt = 1.0 / (a.atol + a.rtol * fabs(y[j]));
                 const double t = ((hs * 0.5) * (fb[j] - fa[j])) * wt;
                 err_w = err_w + t * t;
@@ -567,7 +699,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
         double s1 = 0.0, s2 = 0.0;
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int k = w + NW * j;
+            const int k = species_base(w) + NW * j;
             if (k < NSP) {
                 const double y_in = a.qf[(3 + k) * a.P + col];
                 s1 = s1 + rho * th->h298[k] * (y[j] - y_in) / dt;
@@ -579,7 +711,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
     if (!ok || !owner) return;
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        const int k = w + NW * j;
+        const int k = species_base(w) + NW * j;
         if (k < NSP) a.qf[(3 + k) * a.P + col] = y[j];
     }
     if (w == 0) {
@@ -599,7 +731,7 @@ __global__ void __launch_bounds__(64 * NW) k_chem_retry(ChemArgs a) {
 hipError_t launch_chem_retry(const ChemArgs &a, int nsp, hipStream_t st) {
     const unsigned nb = unsigned((a.ncells + NC - 1) / NC);
     if (nb == 0) return hipSuccess;
-#define FCFD_CASE(N) if (nsp == N) { hipLaunchKernelGGL((k_chem_retry<N>), dim3(nb), dim3(64 * NW), 0, st, a); return hipGetLastError(); }
+#define FCFD_CASE(N) if (nsp == N) { hipLaunchKernelGGL((k_chem_retry<N>), dim3(nb), dim3(64 * RW), 0, st, a); return hipGetLastError(); }
     FCFD_FOR_EACH_NSP(FCFD_CASE)
 #undef FCFD_CASE
     return hipErrorInvalidValue;
@@ -608,7 +740,7 @@ hipError_t launch_chem_retry(const ChemArgs &a, int nsp, hipStream_t st) {
 hipError_t launch_chem_screen(const ChemArgs &a, int nsp, hipStream_t st) {
     const unsigned nb = unsigned((a.ncells + NC - 1) / NC);
     if (nb == 0) return hipSuccess;
-#define FCFD_CASE(N) if (nsp == N) { hipLaunchKernelGGL((k_chem_screen<N>), dim3(nb), dim3(64 * NW), 0, st, a); return hipGetLastError(); }
+#define FCFD_CASE(N) if (nsp == N) { hipLaunchKernelGGL((k_chem_screen<N>), dim3(nb), dim3(64 * RW), 0, st, a); return hipGetLastError(); }
     FCFD_FOR_EACH_NSP(FCFD_CASE)
 #undef FCFD_CASE
     return hipErrorInvalidValue;

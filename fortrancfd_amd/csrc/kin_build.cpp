@@ -75,25 +75,36 @@ void build_dev_kin(const Mech &m, DevKin &k) {
         k.tb[r] = tb_of[i];
         k.fo[r] = fo_of[i];
     }
-    // scatter lists of the lane-per-cell kernels, over the device rows
-    int ne = 0;
+    // lists of the lane-per-cell kernels, over the device rows
+    int ne = 0, ns = 0;
     const int nchunk = (m.ii + LANE_CHUNK - 1) / LANE_CHUNK;
-    static_assert(sizeof(k.lane_ent0) / sizeof(int) >= (MAXR + LANE_CHUNK - 1) / LANE_CHUNK * LANE_NW + 1,
-                  "lane_ent0 holds one start per chunk and wave");
-    for (int c = 0; c < nchunk; ++c)
-        for (int w = 0; w < LANE_NW; ++w) {
-            k.lane_ent0[c * LANE_NW + w] = ne;
-            for (int r = 0; r < LANE_CHUNK; ++r) {
-                const int row = c * LANE_CHUNK + r;
-                if (row >= m.ii) break;
-                for (int n = 0; n < 6; ++n) {
-                    const int sp = k.nk[row][n];
-                    if (sp >= 0 && sp % LANE_NW == w)
-                        k.lane_ent[ne++] = LaneEnt{sp * LANE_NC * 8, r * LANE_NC * 8, double(k.nu[row][n])};
-                }
+    for (int c = 0; c < nchunk; ++c) {
+        std::vector<std::vector<LaneEnt>> of(size_t(m.kk));
+        for (int r = 0; r < LANE_CHUNK && c * LANE_CHUNK + r < m.ii; ++r)
+            for (int n = 0; n < 6; ++n) {
+                const int row = c * LANE_CHUNK + r, sp = k.nk[row][n];
+                if (sp >= 0) of[size_t(sp)].push_back(LaneEnt{double(k.nu[row][n]), r * LANE_NC * 8, 0});
+            }
+        std::vector<int> order;
+        for (int sp = 0; sp < m.kk; ++sp)
+            if (!of[size_t(sp)].empty()) order.push_back(sp);
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return of[size_t(x)].size() > of[size_t(y)].size(); });
+        std::vector<int> mine[LANE_RW];
+        size_t load[LANE_RW] = {};
+        for (int sp : order) {
+            const int w = int(std::min_element(load, load + LANE_RW) - load);
+            mine[w].push_back(sp);
+            load[w] += of[size_t(sp)].size() + 2;
+        }
+        for (int w = 0; w < LANE_RW; ++w) {
+            k.lane_seg0[c * LANE_RW + w] = ns;
+            for (int sp : mine[w]) {
+                k.lane_seg[ns++] = LaneSeg{sp * LANE_NC * 8, ne, int(of[size_t(sp)].size())};
+                for (const LaneEnt &e : of[size_t(sp)]) k.lane_ent[ne++] = e;
             }
         }
-    k.lane_ent0[nchunk * LANE_NW] = ne;
+    }
+    k.lane_seg0[nchunk * LANE_RW] = ns;
     for (int r = k.nplain0; r < m.ii; ++r) {
         LanePlain &p = k.lane_plain[r];
         p.A = k.A[r];
@@ -103,7 +114,7 @@ void build_dev_kin(const Mech &m, DevKin &k) {
         for (int n = 0; n < 6; ++n) {
             const int sp = k.nk[r][n];
             p.nud[n] = double(k.nu[r][n]);
-            p.off[n] = (unsigned short)((sp >= 0 ? sp : 0) * LANE_NC * 8);
+            p.off[n] = (sp >= 0 ? sp : 0) * LANE_NC * 8;
             if (sp >= 0) (n < 3 ? nr : np) += 1;
             const int a = k.nu[r][n] < 0 ? -k.nu[r][n] : k.nu[r][n];
             pw |= (sp >= 0 ? a : 0) << (2 * n);
@@ -130,10 +141,14 @@ void build_coop_lists(DevKin &k, std::vector<unsigned> &jac) {
     const int ii = k.ii, nb = (ii + 63) / 64;
     bool fits = ii <= COOP_MAXR && k.kk < COOP_EMPTY && k.nfal <= COOP_FAL;
     auto usual = [](double v) { return v == 0.0 || (std::fabs(v) >= 0x1p-700 && std::fabs(v) <= 0x1p60); };
-    for (int f = 0; f < k.nfal; ++f) fits = fits && usual(k.fpar[f][2]) && usual(k.fpar[f][6]);
+    k.usual = 1;
+    for (int f = 0; f < k.nfal; ++f)
+        if (!usual(k.fpar[f][2]) || !usual(k.fpar[f][6])) k.usual = 0;
+    for (int r = 0; r < ii; ++r)
+        if (!usual(k.E[r]) || !(std::fabs(k.E[r]) <= 0x1p22 && std::fabs(k.B[r]) <= 0x1p20)) k.usual = 0;
+    fits = fits && k.usual;
     for (int r = 0; r < ii; ++r) {
         const int *nu = k.nu[r], *nk = k.nk[r];
-        fits = fits && usual(k.E[r]);
         fits = fits && std::abs(k.nus[r]) <= 3 && nk[0] >= 0 && nk[3] >= 0 && (nk[1] >= 0 || nk[2] < 0) &&
                (nk[4] >= 0 || nk[5] < 0) && (k.tb[r] < 0 || k.ntbs[k.tb[r]] <= COOP_TB);
         bool pow = false;
