@@ -166,6 +166,7 @@ int ensure_dev_tables(const fcfd_mech *cm) {
         HIP_TRY(hipMemcpy(lists.p, jac.data(), jac.size() * sizeof(unsigned), hipMemcpyHostToDevice));
         k->coop_jac = static_cast<const unsigned *>(lists.p);
     }
+    const bool coop = k->coop != 0;
     HIP_TRY(hipMalloc(&kin.p, sizeof(DevKin)));
     HIP_TRY(hipMemcpy(kin.p, k.get(), sizeof(DevKin), hipMemcpyHostToDevice));
     HIP_TRY(hipMalloc(&counter.p, sizeof(unsigned int)));
@@ -174,6 +175,7 @@ int ensure_dev_tables(const fcfd_mech *cm) {
     m->d_kin = kin.p;
     m->d_counter = static_cast<unsigned int *>(counter.p);
     m->d_lists = lists.p;
+    m->coop = coop;
     th.p = kin.p = counter.p = lists.p = nullptr;
     m->device = dev;
     return FCFD_OK;
@@ -472,6 +474,7 @@ hipError_t enqueue_aux(fcfd_ctx *c, double dt, const double *dt_dev, double time
 hipError_t enqueue_source(fcfd_ctx *c, double dt, const double *dt_dev, bool want_hrr) {
     ChemArgs a{};
     a.thermo = c->thermo; a.kin = static_cast<const DevKin *>(c->mech->d_kin); a.counter = c->d_counter;
+    a.coop = c->mech->coop;
     a.ncells = c->nblk * c->ncell; a.rtol = c->o.rtol; a.atol = c->o.atol;
     a.qf = c->qf; a.P = c->P; a.ncell = c->ncell; a.lv = c->lv; a.S = c->S;
     a.dt = dt; a.dt_dev = dt_dev; a.stats = c->d_stats; a.order = c->d_order; a.hmem = c->d_hmem;
@@ -479,11 +482,12 @@ hipError_t enqueue_source(fcfd_ctx *c, double dt, const double *dt_dev, bool wan
     a.layout = 0;
     const int chem_wg = c->chem_wg > 0 ? c->chem_wg : chem_workgroups(c->mech);
     a.route = c->d_accepted;
-    a.f0 = c->d_f0;
     const int n = c->nblk * c->ncell;
+    const int limit = coop_limit(a, chem_wg, c->kk);
+    a.f0 = n > limit ? c->d_f0 : nullptr;
     // explicit screen, one cell per lane: quiescent cells are final, the rest form the stiff list
     hipError_t e = timed(c, 6, [&]() {
-        hipError_t e2 = launch_zero_u32(c->d_list_n, c->stream);
+        hipError_t e2 = launch_zero_u32(c->d_list_n, c->stream, c->d_list2_n);
         if (e2 != hipSuccess) return e2;
         a.stiff = c->d_list;
         a.stiff_n = c->d_list_n;
@@ -491,39 +495,45 @@ hipError_t enqueue_source(fcfd_ctx *c, double dt, const double *dt_dev, bool wan
     });
     if (e != hipSuccess) return e;
     // a long stiff list (the cold region failing the screen at once) first gets the explicit
-    // half-step retry lane-per-cell; what remains, or a short list unchanged, is d_list2
-    e = timed(c, 8, [&]() {
-        hipError_t e2 = launch_zero_u32(c->d_list2_n, c->stream);
-        if (e2 != hipSuccess) return e2;
-        ChemArgs r = a;
-        r.list = c->d_list;
-        r.list_n = c->d_list_n;
-        r.stiff = c->d_list2;
-        r.stiff_n = c->d_list2_n;
-        r.retry_done = c->d_retry;
-        r.coop_max = chem_coop_max(chem_wg, c->kk);
-        return launch_chem_retry(r, c->kk, c->stream);
-    });
-    if (e != hipSuccess) return e;
-    a.retry_done = c->d_retry;
+    // half-step retry lane-per-cell; what remains, or a short list unchanged, is d_list2.  In a domain
+    // whose every list is short the retry is left to the eight-wave integrator without asking (a launch
+    // that only copies the list costs 4.5 us).
+    int *list = c->d_list;
+    unsigned *list_n = c->d_list_n;
+    if (n > limit) {
+        e = timed(c, 8, [&]() {
+            ChemArgs r = a;
+            r.list = c->d_list;
+            r.list_n = c->d_list_n;
+            r.stiff = c->d_list2;
+            r.stiff_n = c->d_list2_n;
+            r.retry_done = c->d_retry;
+            r.coop_max = limit;
+            return launch_chem_retry(r, c->kk, c->stream);
+        });
+        if (e != hipSuccess) return e;
+        a.retry_done = c->d_retry;
+        list = c->d_list2;
+        list_n = c->d_list2_n;
+    }
     if (c->sur) {
         fcfd_surrogate *s = c->sur;
         e = timed(c, 5, [&]() {
             FeatArgs fa{};
             fa.layout = 0; fa.n = n; fa.qf = c->qf; fa.P = c->P; fa.ncell = c->ncell; fa.lv = c->lv; fa.S = c->S;
             fa.dt_dev = dt_dev; fa.dt = dt;
-            hipError_t e2 = s->network(fa, c->d_list2, c->d_list2_n, n, c->stream);
+            hipError_t e2 = s->network(fa, list, list_n, n, c->stream);
             if (e2 != hipSuccess) return e2;
             ApplyArgs ap{};
             ap.layout = 0; ap.qf = c->qf; ap.P = c->P; ap.ncell = c->ncell; ap.lv = c->lv; ap.S = c->S;
             ap.route = c->d_accepted;
-            return s->accept(ap, a, c->d_list2, c->d_list2_n, n, c->stream);
+            return s->accept(ap, a, list, list_n, n, c->stream);
         });
         if (e != hipSuccess) return e;
         e = timed(c, 3, [&]() { return s->fallback(a, chem_wg, c->stream); });
     } else {
-        a.list = c->d_list2;
-        a.list_n = c->d_list2_n;
+        a.list = list;
+        a.list_n = list_n;
         a.skip_explicit = 1;
         e = timed(c, 3, [&]() { return launch_chem(a, c->kk, chem_wg, c->stream); });
     }
@@ -1278,6 +1288,7 @@ int fcfd_chem_batch(const fcfd_mech *m, const fcfd_opts *o, int n, const double 
     if (int rc = ensure_dev_tables(m)) return rc;
     ChemArgs a{};
     a.thermo = m->d_thermo; a.kin = static_cast<const DevKin *>(m->d_kin); a.counter = m->d_counter;
+    a.coop = m->coop;
     a.ncells = n; a.rtol = o->rtol; a.atol = o->atol;
     a.b_rho = rho; a.b_dt = dt; a.b_T = T; a.b_y = Y;
     a.stats = reinterpret_cast<ChemCellStats *>(stats);
@@ -1328,6 +1339,7 @@ int fcfd_chem_batch_noalloc(const fcfd_mech *m, const fcfd_opts *o, int n, const
     if (int rc = noalloc_scratch(dev, &base)) return rc;
     ChemArgs a{};
     a.thermo = m->d_thermo; a.kin = static_cast<const DevKin *>(m->d_kin);
+    a.coop = m->coop;
     a.counter = reinterpret_cast<unsigned int *>(base);                 // work-queue head
     a.ncells = n; a.rtol = o->rtol; a.atol = o->atol;
     a.b_rho = rho; a.b_dt = dt; a.b_T = T; a.b_y = Y;

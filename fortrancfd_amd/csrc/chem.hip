@@ -713,8 +713,11 @@ __global__ void __launch_bounds__(64) k_rates(const DevThermo *__restrict__ th, 
     }
 }
 
-__global__ void k_zero_counter(unsigned int *c) {
-    if (threadIdx.x == 0) *c = 0u;
+__global__ void k_zero_counter(unsigned int *c, unsigned int *d) {
+    if (threadIdx.x == 0) {
+        *c = 0u;
+        if (d) *d = 0u;
+    }
 }
 
 __global__ void k_scale_scalar(const double *in, double *out, double f) {
@@ -724,15 +727,19 @@ __global__ void k_scale_scalar(const double *in, double *out, double f) {
 // Stable partition of a work list by the cells' attempt counts (steps + rejects) of the previous
 // integration: first those with at least CH_HEAVY, then the rest.  A launch lasts as long as its
 // slowest cell, and the cells that were slow in the last step are, near a flame, the slow ones in
-// this step; started first, they do not wait behind a queue of cheap cells.  One workgroup.
+// this step; started first, they do not wait behind a queue of cheap cells.  One workgroup.  Clears the
+// integrator's queue head on the way.
 constexpr int CH_HEAVY = 4;
 
 __global__ void __launch_bounds__(1024) k_heavy_first(const int *list, const unsigned *list_n,
-                                                      const ChemCellStats *stats, int *out) {
+                                                      const ChemCellStats *stats, int *out, unsigned *counter) {
     __shared__ unsigned wcount[16], woff[16], base, total;
     const int n = int(*list_n);
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    if (t == 0) base = 0;
+    if (t == 0) {
+        base = 0;
+        *counter = 0;
+    }
     __syncthreads();
     for (int pass = 0; pass < 2; ++pass) {
         for (int i0 = 0; i0 < n; i0 += 1024) {
@@ -769,8 +776,8 @@ hipError_t launch_scale_scalar(const double *in, double *out, double f, hipStrea
     return hipGetLastError();
 }
 
-hipError_t launch_zero_u32(unsigned *p, hipStream_t st) {
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, p);
+hipError_t launch_zero_u32(unsigned *p, hipStream_t st, unsigned *q) {
+    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, p, q);
     return hipGetLastError();
 }
 
@@ -816,25 +823,27 @@ hipError_t launch_chem_full(ChemArgs a, int nsp, int n_workgroups, int *list, un
 // n_workgroups one-wave workgroups (five per CU by default) for long lists; two fifths as many eight-wave
 // workgroups -- two per CU, what its LDS and registers hold -- for lists of at most a.coop_max cells (the
 // tuned factor, default 8, times n_workgroups).  Up to coop_max the launch is set by its slowest cells,
-// which eight waves take through a step several times as fast as one.  Both kernels are launched; the one
-// whose mode does not match the list length on the device returns at once.
+// which eight waves take through a step several times as fast as one.  Both kernels are launched, and the
+// one whose mode does not match the list length on the device returns at once; where no list can be long, or
+// the mechanism does not suit the eight-wave kernel, only the one that can run (a launch that returns at
+// once costs 4.5 us, 4 % of a small domain's call).
 hipError_t launch_chem(const ChemArgs &a0, int nsp, int n_workgroups, hipStream_t st) {
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, a0.counter);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    hipError_t e;
     ChemArgs a = a0;
-    a.coop_max = chem_coop_max(n_workgroups, nsp);
+    a.coop_max = coop_limit(a, n_workgroups, nsp);
     if (a.order && a.list && a.list_n && a.stats && a.layout == 0) {
-        hipLaunchKernelGGL(k_heavy_first, dim3(1), dim3(1024), 0, st, a.list, a.list_n, a.stats, a.order);
+        hipLaunchKernelGGL(k_heavy_first, dim3(1), dim3(1024), 0, st, a.list, a.list_n, a.stats, a.order, a.counter);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         a.list = a.order;
+    } else if ((e = launch_zero_u32(a.counter, st)) != hipSuccess) {
+        return e;
     }
     const int nwg1 = std::min(n_workgroups, a.ncells);
     const int nwg8 = std::min(std::max(2 * n_workgroups / 5, 1), a.ncells);
     if (nwg1 <= 0) return hipSuccess;
 #define FCFD_CASE(N) if (nsp == N) { \
-        if ((e = launch_chem_coop(a, nsp, nwg8, st)) != hipSuccess) return e; \
-        hipLaunchKernelGGL((k_chem<N>), dim3(nwg1), dim3(64), 0, st, a); \
+        if (a.coop && (e = launch_chem_coop(a, nsp, nwg8, st)) != hipSuccess) return e; \
+        if (a.ncells > a.coop_max) hipLaunchKernelGGL((k_chem<N>), dim3(nwg1), dim3(64), 0, st, a); \
         return hipGetLastError(); }
     FCFD_FOR_EACH_NSP(FCFD_CASE)
 #undef FCFD_CASE

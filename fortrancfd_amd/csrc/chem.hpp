@@ -149,6 +149,7 @@ struct ChemArgs {
     int *route;                  // optional per-cell route: 2 explicit step over dt, 3 two explicit half
                                  // steps, 1 surrogate, 0 implicit (SDIRK) integrator
     int layout;                  // 0: domain, 1: batch
+    int coop;                    // 1: the mechanism suits the eight-wave integrator (fcfd_mech::coop)
     int coop_max;                // set by launch_chem: lists up to this length run eight waves per cell
     // optional (domain layout with stats): buffer of the list's capacity that receives the list
     // reordered with the cells whose previous integration took the most attempts first
@@ -178,7 +179,9 @@ hipError_t launch_chem_retry(const ChemArgs &a, int nsp, hipStream_t st);
 // Longest list that the eight-wave integrator mode takes: the tuned factor (default 8) times the
 // workgroup count (api.hip).
 int chem_coop_max(int n_workgroups, int nsp);
-hipError_t launch_zero_u32(unsigned *p, hipStream_t st);
+// The same for these cells: -1 where the mechanism does not suit that mode.
+inline int coop_limit(const ChemArgs &a, int n_workgroups, int nsp) { return a.coop ? chem_coop_max(n_workgroups, nsp) : -1; }
+hipError_t launch_zero_u32(unsigned *p, hipStream_t st, unsigned *q = nullptr);      // *p = 0, *q = 0
 // *out = f * *in on the device (one thread), e.g. the half step of Strang splitting.
 hipError_t launch_scale_scalar(const double *in, double *out, double f, hipStream_t st);
 // CKWYR / CKCDYR (cklib.f:9107-9204, 1422-1541) on n states with the integrator's own rate code:

@@ -8,7 +8,7 @@
 namespace fcfd {
 
 // The integrator mode for a list of n cells: eight waves per cell, else one.
-__device__ __forceinline__ bool coop_list(const ChemArgs &a, int n) { return n <= a.coop_max && a.kin->coop != 0; }
+__device__ __forceinline__ bool coop_list(const ChemArgs &a, int n) { return n <= a.coop_max; }
 
 // x**n by binary powering (the product order of the CPU restatement); negative n as 1 / x**(-n).
 // Written without recursion so it inlines: a call from a kernel holding hundreds of live registers

@@ -84,6 +84,7 @@ struct fcfd_mech {
     fcfd::DevThermo *d_thermo = nullptr;
     void *d_kin = nullptr;               // fcfd::DevKin
     void *d_lists = nullptr;             // the eight-wave integrator's Jacobian lists (chem.hpp)
+    bool coop = false;                   // the mechanism suits that integrator
     unsigned int *d_counter = nullptr;   // work queue of batched chemistry calls
     int *d_list = nullptr;               // stiff-cell list of batched chemistry calls (grown on demand)
     unsigned *d_list_n = nullptr;

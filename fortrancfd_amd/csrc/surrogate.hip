@@ -376,6 +376,7 @@ int fcfd_sur_infer_batch(fcfd_surrogate *s, const fcfd_opts *o, int n, const dou
     HIP_TRY(s->reserve(npad, false));
     ChemArgs ca{};
     ca.thermo = s->mech->d_thermo; ca.kin = static_cast<const DevKin *>(s->mech->d_kin); ca.counter = s->mech->d_counter;
+    ca.coop = s->mech->coop;
     ca.ncells = n; ca.rtol = o->rtol; ca.atol = o->atol;
     ca.b_rho = rho; ca.b_dt = dt; ca.b_T = T; ca.b_y = Y;
     ca.stats = reinterpret_cast<ChemCellStats *>(stats);
