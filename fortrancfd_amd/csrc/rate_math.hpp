@@ -30,6 +30,13 @@ __device__ __forceinline__ CSeries *get_series() {
     return k;
 }
 
+// a b + k with k a scalar operand (left to itself the compiler moves k into the destination first)
+__device__ __forceinline__ double fma_k(double a, double b, double k) {
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(k));
+    return r;
+}
+
 // exp of the two-term value x + xl with fm_exp's bits (arguments beyond +-1000 give infinity or 0)
 __device__ __forceinline__ double exp2term(CSeries *k, double x, double xl) {
     const double xc = __builtin_fmin(__builtin_fmax(x, -k->limit), k->limit);
@@ -40,7 +47,7 @@ __device__ __forceinline__ double exp2term(CSeries *k, double x, double xl) {
     const double rl = r1 - (rh - r0);
     double p = k->exp[0];
 #pragma unroll
-    for (int i = 1; i < 13; ++i) p = __builtin_fma(p, rh, k->exp[i]);
+    for (int i = 1; i < 13; ++i) p = fma_k(p, rh, k->exp[i]);
     const double q = (rh * rh) * p;
     const double s = 1.0 + rh;
     const double e = rh - (s - 1.0);
@@ -55,7 +62,7 @@ __device__ __forceinline__ double exp_near(CSeries *k, double x) {
     const double rl = r1 - (rh - r0);
     double p = k->exp[0];
 #pragma unroll
-    for (int i = 1; i < 13; ++i) p = __builtin_fma(p, rh, k->exp[i]);
+    for (int i = 1; i < 13; ++i) p = fma_k(p, rh, k->exp[i]);
     const double q = (rh * rh) * p;
     const double s = 1.0 + rh;
     const double e = rh - (s - 1.0);
@@ -84,7 +91,7 @@ __device__ __forceinline__ double log_dd_rate(CSeries *k, double x, double &lo) 
     const double z = sh * sh;
     double p = k->log[0];
 #pragma unroll
-    for (int i = 1; i < 12; ++i) p = __builtin_fma(p, z, k->log[i]);
+    for (int i = 1; i < 12; ++i) p = fma_k(p, z, k->log[i]);
     const double small = 2.0 * sl + ((sh * z) * p + 2.0 * z * sl);
     const double ed = double(e);
     const double ph = ed * k->ln2_hi;
