@@ -11,17 +11,16 @@ constexpr int LANE_CHUNK = 7 * LANE_RW;   // reaction rows between two barriers 
 constexpr int LANE_NC = 64;      // cells per workgroup of the lane-per-cell kernels
 
 // A row of the branch-free range (nplain0 .. ii-1) as the lane-per-cell kernels read it, with one
-// row index for the whole wave: coefficients as doubles, and the species of each present slot as the
-// byte offset k * LANE_NC * 8 of its row in a species-major [k][LANE_NC] LDS block.  Reactant slots
-// are 0 .. nr-1, product slots 3 .. 3+np-1 (build_dev_kin admits only rows stored that way).
+// row index for the whole wave: coefficients as doubles, and the species of each slot as the byte
+// offset k * LANE_NC * 8 of its row in a species-major [k][LANE_NC] LDS block (an empty slot: coefficient 0,
+// the row after the last species).
 struct LanePlain {
     double A, B, E;
     double nud[6];
     int off[6];
     int bits;                    // LP_* fields
 };
-constexpr int LP_NR = 0;         // bits 0-1: reactant slots (1-3)
-constexpr int LP_NP = 2;         // bits 2-3: product slots (0-3)
+// LanePlain::bits
 constexpr int LP_REV = 1 << 4;   // reverse rate from the equilibrium constant
 constexpr int LP_ARR0 = 1 << 5;  // B = E = 0
 constexpr int LP_NUS = 6;        // bits 6-8: coefficient sum + 3

@@ -18,11 +18,11 @@
 // what.  Species-wise work (thermo, state update, norms) is split over the first NW = 8 waves by k mod
 // NW; cell-wise scalars (T, sums) are combined through LDS in wave order, by every wave.
 //
-// Bound: the issue of one SIMD's four waves.  A plain row takes some 120 vector operations (two
-// exponentials, a division), a fall-off row 500; 325 rows are 62k cycles of a SIMD, of which a right-hand
-// side took 100k, and 35k more go to the species' terms and the sums.  LDS (143 KB) holds one workgroup
-// per compute unit; 128 registers a lane allow its 16 waves.  65,536 cells (four rounds of 256
-// workgroups): 682 us a launch, 510 cells: 181 us.  Eight waves with 32-row chunks, one fixed row in
+// Bound: the issue of one SIMD's four waves.  A plain row takes some 110 vector operations (two
+// exponentials, a division), a fall-off row 500.  LDS (144 KB) holds one workgroup per compute unit; 128
+// registers a lane allow its 16 waves.  65,536 cells (four rounds of 256 workgroups): 574 us a launch, 510
+// cells: 155 us.  (682 and 181 while the series' constants went through vector registers and empty slots
+// were selected away.)  Eight waves with 32-row chunks, one fixed row in
 // eight each, and table reads that went through the vector cache at each branch took 1,098 and 334 us.
 #include <algorithm>
 
@@ -42,8 +42,8 @@ constexpr int CH = LANE_CHUNK; // reaction rows per chunk
 
 template <int NSP>
 struct LaneShared {
-    double C[NSP * NC];        // concentrations, mol/cm^3
-    double G[NSP * NC];        // S/R - H/RT
+    double C[(NSP + 1) * NC];  // concentrations, mol/cm^3; the last row, for empty slots, is 1
+    double G[(NSP + 1) * NC];  // S/R - H/RT; the last row is 0
     double W[NSP * NC];        // production rates
     double Q[CH * NC];         // rates of progress (forward minus reverse) of the current chunk; outside
                                // the reaction loop, the per-wave values of cross-wave sums
@@ -153,13 +153,11 @@ __device__ __forceinline__ double lane_row_q(CKin *K, CSeries *ks, int i, const 
 }
 
 // reaction_plain (chem_device.hpp) for a row the whole wave evaluates, as forward minus reverse rate of
-// progress: the same operations, with the slot counts, coefficient
-// powers and flags of K->lane_plain taken as scalar branches instead of selects, the species rows
-// read at byte offsets from this lane's column of the C and G blocks, and pfac**nus from the lane's
-// PF column.  Multiplications by exactly 1.0 that reaction_plain makes for empty slots are skipped
-// (they do not change a value).
-__device__ __forceinline__ double ipow_u(double x, int m) {      // ipow3 for a wave-uniform m >= 1
-    if (m == 1) return x;
+// progress: the same operations, with the powers and flags
+// of K->lane_plain taken as scalar branches instead of selects, the species rows read at byte offsets
+// from this lane's column of the C and G blocks, and pfac**nus from the lane's PF column.
+__device__ __forceinline__ double ipow_u(double x, int m) {      // ipow3 for a wave-uniform m; 0 only for x = 1
+    if (m <= 1) return x;
     const double x2 = x * x;
     return m == 2 ? x2 : x * x2;
 }
@@ -173,21 +171,15 @@ __device__ __forceinline__ double lane_plain_q(CLanePlain *L, CSeries *ks, const
     const double nud[6] = {L->nud[0], L->nud[1], L->nud[2], L->nud[3], L->nud[4], L->nud[5]};
     const int off[6] = {L->off[0], L->off[1], L->off[2], L->off[3], L->off[4], L->off[5]};
     if (bits & LP_DEAD) return 0.0;
-    const int nr = (bits >> LP_NR) & 3, np = (bits >> LP_NP) & 3;
-    // concentrations and S/R - H/RT of the filled slots (G follows C at a constant distance)
-    double c[6] = {}, g[6] = {};
-    auto read = [&](int n) {
+    // concentrations and S/R - H/RT of the slots (G follows C at a constant distance); an empty slot reads the
+    // row that changes nothing: coefficient 0, concentration 1
+    double c[6], g[6];
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
         const char *at = Cb + off[n];
         c[n] = *reinterpret_cast<const double *>(at);
         g[n] = *reinterpret_cast<const double *>(at + dG);
-    };
-    read(0);
-    if (nr >= 2) read(1);
-    if (nr >= 3) read(2);
-    if (np >= 1) read(3);
-    if (np >= 2) read(4);
-    if (np >= 3) read(5);
-    auto C = [&](int n) { return c[n]; };
+    }
     double kf = A;
     if (!(bits & LP_ARR0)) kf = kf * exp_near(ks, B * tp.logT - over(E, tp, usual));
     double kr = 0.0;
@@ -195,32 +187,18 @@ __device__ __forceinline__ double lane_plain_q(CLanePlain *L, CSeries *ks, const
         // reaction_plain starts from 0.0 + t0; the two differ at most in the sign of a zero sum,
         // which the test s != 0 and exp(+-0) = 1 do not see
         double s = nud[0] * g[0];
-        if (nr >= 2) s = s + nud[1] * g[1];
-        if (nr >= 3) s = s + nud[2] * g[2];
-        if (np >= 1) s = s + nud[3] * g[3];
-        if (np >= 2) s = s + nud[4] * g[4];
-        if (np >= 3) s = s + nud[5] * g[5];
+#pragma unroll
+        for (int n = 1; n < 6; ++n) s = s + nud[n] * g[n];
         double eqk = exp_near(ks, fmin(s, exparg));      // (1 for s = 0)
         eqk = eqk * Pf[((bits >> LP_NUS) & 7) * NC];
         kr = kf / fmax(eqk, small);
     }
-    double qf, qr = kr;
-    if (!(bits & LP_POW)) {
-        qf = kf * C(0);
-        if (nr >= 2) qf = qf * C(1);
-        if (nr >= 3) qf = qf * C(2);
-        if (np >= 1) qr = kr * C(3);
-        if (np >= 2) qr = qr * C(4);
-        if (np >= 3) qr = qr * C(5);
-    } else {
+    if (bits & LP_POW) {
         const int pw = bits >> LP_PW;
-        qf = kf * ipow_u(C(0), pw & 3);
-        if (nr >= 2) qf = qf * ipow_u(C(1), (pw >> 2) & 3);
-        if (nr >= 3) qf = qf * ipow_u(C(2), (pw >> 4) & 3);
-        if (np >= 1) qr = kr * ipow_u(C(3), (pw >> 6) & 3);
-        if (np >= 2) qr = qr * ipow_u(C(4), (pw >> 8) & 3);
-        if (np >= 3) qr = qr * ipow_u(C(5), (pw >> 10) & 3);
+#pragma unroll
+        for (int n = 0; n < 6; ++n) c[n] = ipow_u(c[n], (pw >> (2 * n)) & 3);
     }
+    const double qf = kf * c[0] * c[1] * c[2], qr = kr * c[3] * c[4] * c[5];
     return qf - qr;
 }
 
@@ -420,7 +398,12 @@ __global__ void __launch_bounds__(64 * RW) k_chem_screen(ChemArgs a) {
     const bool owner = live && int(threadIdx.x & 63) < NC;
     const int c = live ? cell : cell0;          // columns past the end shadow a live cell
     double *slot = sh.Q;
-    if (threadIdx.x < 2) sh.next[threadIdx.x] = 0;      // (barriers before the first rows)
+    // (barriers follow before the first rows)
+    if (threadIdx.x < 2) sh.next[threadIdx.x] = 0;
+    if (w == 0) {
+        sh.C[NSP * NC + lane] = 1.0;
+        sh.G[NSP * NC + lane] = 0.0;
+    }
 
     long col = 0;
     double rho_si, dt, T0;
@@ -599,7 +582,12 @@ __global__ void __launch_bounds__(64 * RW) k_chem_retry(ChemArgs a) {
     const bool owner = live && int(threadIdx.x & 63) < NC;
     const int cell = a.list[live ? item : item0];   // columns past the end shadow a live cell
     double *slot = sh.Q;
-    if (threadIdx.x < 2) sh.next[threadIdx.x] = 0;      // (barriers before the first rows)
+    // (barriers follow before the first rows)
+    if (threadIdx.x < 2) sh.next[threadIdx.x] = 0;
+    if (w == 0) {
+        sh.C[NSP * NC + lane] = 1.0;
+        sh.G[NSP * NC + lane] = 0.0;
+    }
 
     const int b = cell / a.ncell, i = cell % a.ncell;
     const long col = long(b) * a.S + a.lv + i;

@@ -110,17 +110,16 @@ void build_dev_kin(const Mech &m, DevKin &k) {
         p.A = k.A[r];
         p.B = k.B[r];
         p.E = k.E[r];
-        int nr = 0, np = 0, pw = 0, big = 0;
+        int pw = 0, big = 0;
         for (int n = 0; n < 6; ++n) {
             const int sp = k.nk[r][n];
-            p.nud[n] = double(k.nu[r][n]);
-            p.off[n] = (sp >= 0 ? sp : 0) * LANE_NC * 8;
-            if (sp >= 0) (n < 3 ? nr : np) += 1;
+            p.nud[n] = sp >= 0 ? double(k.nu[r][n]) : 0.0;
+            p.off[n] = (sp >= 0 ? sp : m.kk) * LANE_NC * 8;
             const int a = k.nu[r][n] < 0 ? -k.nu[r][n] : k.nu[r][n];
             pw |= (sp >= 0 ? a : 0) << (2 * n);
             if (sp >= 0 && a > 1) big = 1;
         }
-        p.bits = (nr << LP_NR) | (np << LP_NP) | (k.rev[r] ? LP_REV : 0) | (k.arr0[r] ? LP_ARR0 : 0) |
+        p.bits = (k.rev[r] ? LP_REV : 0) | (k.arr0[r] ? LP_ARR0 : 0) |
                  ((k.nus[r] + 3) << LP_NUS) | (big ? LP_POW : 0) | (pw << LP_PW) | (k.nu[r][0] == 0 ? LP_DEAD : 0);
     }
     for (int t = 0; t < k.nthb; ++t) {
