@@ -643,11 +643,15 @@ __device__ __forceinline__ void serve_rates(const DevKin *__restrict__ K, Cell<N
     }
 }
 
+// The compiler's own lane write (clang has no builtin for it): a vector instruction may read a scalar register
+// that another vector instruction wrote only two wait states later, and the compiler provides them for
+// instructions that it knows, not inside inline assembly.
+extern "C" __device__ int fcfd_writelane(int v, int k, int old) __asm("llvm.amdgcn.writelane.i32");
+
 // v, the same in all lanes, into lane k of x
 __device__ __forceinline__ double put_lane(double x, double v, const int k) {
-    int lo = __double2loint(x), hi = __double2hiint(x);
-    asm("v_writelane_b32 %0, %1, %2" : "+v"(lo) : "s"(__double2loint(v)), "n"(k));
-    asm("v_writelane_b32 %0, %1, %2" : "+v"(hi) : "s"(__double2hiint(v)), "n"(k));
+    const int lo = fcfd_writelane(__double2loint(v), k, __double2loint(x));
+    const int hi = fcfd_writelane(__double2hiint(v), k, __double2hiint(x));
     return __hiloint2double(hi, lo);
 }
 
