@@ -88,7 +88,7 @@ struct DevKin {
     // Third bodies of a row: species, a byte each (COOP_EMPTY: none), and efficiency - 1 (0)
     unsigned coop_tbk[COOP_TB / 4][MAXR];
     double coop_tba[COOP_TB][MAXR];
-    // 1: the mechanism suits that integrator: at most COOP_MAXR rows, |coefficients| and their sums at
+    // 1: the mechanism suits that integrator (else its short lists take k_chem's four-wave mode): at most COOP_MAXR rows, |coefficients| and their sums at
     // most 3, no negative product coefficient, no gap before a filled slot, at most COOP_TB third bodies
     // and COOP_FAL fall-off rows, constants that over() may divide by T's reciprocal.
     int coop;
@@ -149,7 +149,7 @@ struct ChemArgs {
                                  // steps, 1 surrogate, 0 implicit (SDIRK) integrator
     int layout;                  // 0: domain, 1: batch
     int coop;                    // 1: the mechanism suits the eight-wave integrator (fcfd_mech::coop)
-    int coop_max;                // set by launch_chem: lists up to this length run eight waves per cell
+    int coop_max;                // set by launch_chem: lists up to this length run several waves per cell
     // optional (domain layout with stats): buffer of the list's capacity that receives the list
     // reordered with the cells whose previous integration took the most attempts first
     int *order;
@@ -165,7 +165,8 @@ struct ChemArgs {
 };
 
 // SDIRK integrator over all cells or over a work list (persistent grid): one cell per wave for long
-// lists, one cell per eight-wave workgroup (launch_chem_coop) for short ones.
+// lists, one cell per workgroup for short ones: eight waves (launch_chem_coop), or four for a mechanism
+// beyond that kernel's tables.
 hipError_t launch_chem_coop(const ChemArgs &a, int nsp, int nwg, hipStream_t st);
 hipError_t launch_chem(const ChemArgs &a, int nsp, int n_workgroups, hipStream_t st);
 // Lane-per-cell explicit screen over cells 0 .. ncells: accepted cells are final, the others are
@@ -175,11 +176,9 @@ hipError_t launch_chem_screen(const ChemArgs &a, int nsp, hipStream_t st);
 // a.coop_max: accepted cells are final, the others go to a.stiff (a.stiff_n must be zero before
 // the launch) and *a.retry_done = 1; a shorter list is copied to a.stiff unchanged, *a.retry_done = 0.
 hipError_t launch_chem_retry(const ChemArgs &a, int nsp, hipStream_t st);
-// Longest list that the eight-wave integrator mode takes: the tuned factor (default 8) times the
-// workgroup count (api.hip).
+// Longest list that gets a workgroup per cell: the tuned factor (default 8) times the workgroup count
+// (api.hip).
 int chem_coop_max(int n_workgroups, int nsp);
-// The same for these cells: -1 where the mechanism does not suit that mode.
-inline int coop_limit(const ChemArgs &a, int n_workgroups, int nsp) { return a.coop ? chem_coop_max(n_workgroups, nsp) : -1; }
 hipError_t launch_zero_u32(unsigned *p, hipStream_t st, unsigned *q = nullptr);      // *p = 0, *q = 0
 // *out = f * *in on the device (one thread), e.g. the half step of Strang splitting.
 hipError_t launch_scale_scalar(const double *in, double *out, double f, hipStream_t st);

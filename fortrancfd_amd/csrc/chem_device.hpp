@@ -7,7 +7,7 @@
 
 namespace fcfd {
 
-// The integrator mode for a list of n cells: eight waves per cell, else one.
+// The integrator mode for a list of n cells: several waves per cell, else one.
 __device__ __forceinline__ bool coop_list(const ChemArgs &a, int n) { return n <= a.coop_max; }
 
 // x**n by binary powering (the product order of the CPU restatement); negative n as 1 / x**(-n).

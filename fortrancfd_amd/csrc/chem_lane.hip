@@ -553,7 +553,7 @@ __global__ void __launch_bounds__(64 * RW) k_chem_screen(ChemArgs a) {
 // Accepted cells are final (state, heat release, stats {2, 0, 0, 0}, step-size memory 0); the
 // others go to a.stiff (*a.stiff_n zero before the launch) for the implicit integrator, which
 // *a.retry_done = 1 tells to skip its own retry.  A list of at most a.coop_max cells is copied to
-// a.stiff unchanged with *a.retry_done = 0: the integrator then runs it eight waves per cell and
+// a.stiff unchanged with *a.retry_done = 0: the integrator then runs it several waves per cell and
 // retries each cell itself.  Domain layout only.
 template <int NSP>
 __global__ void __launch_bounds__(64 * RW) k_chem_retry(ChemArgs a) {

@@ -309,7 +309,8 @@ class Solver:
 
     def set_chem_workgroups(self, n):
         """Grid of the implicit integrator (0: default): n one-wave workgroups for lists longer
-        than 8 n cells, else 2 n / 5 eight-wave workgroups."""
+        than 8 n cells, else 2 n / 5 eight-wave workgroups (n / 4 four-wave ones for a mechanism
+        beyond the eight-wave kernel's tables)."""
         _check(lib().fcfd_set_chem_workgroups(self.handle, C.c_int(n)))
 
     def source_accepted(self):

@@ -226,8 +226,8 @@ int fcfd_set_timing(fcfd_ctx *c, int enable);
  * defaults.  Keys: "flux_variant" (WENO5 + HLLC advection flux: register budget for four waves
  * per SIMD with 1, three with 0 or 2), "stage_variant" (stage update: four waves per SIMD with 1,
  * three with 0, 2 or 3), "chem_wg_per_cu" (implicit-integrator workgroups per CU, default 5),
- * "chem_four_wave_factor" (eight waves per cell -- four when the key was named -- for lists of at most
- * factor x workgroups cells, default 8), "chem_lu" (accepted and without effect: it chose between
+ * "chem_four_wave_factor" (several waves per cell for lists of at most factor x workgroups cells, default
+ * 8: eight waves, or four for a mechanism that the eight-wave kernel's tables do not hold), "chem_lu" (accepted and without effect: it chose between
  * factorisations of the same bits, of which one is left; default 2).  fcfd_set_launch overrides one entry for the mechanisms of nsp species (every context
  * re-captures its step graph); fcfd_load_tuning reloads the table (NULL: the default file). */
 int fcfd_set_launch(const char *key, int nsp, int value);
@@ -349,7 +349,8 @@ int fcfd_set_surrogate(fcfd_ctx *c, fcfd_surrogate *s);
  * with 0. */
 int fcfd_source_accepted(fcfd_ctx *c, int *per_cell, int *n_fallback);
 /* Grid of the FP64 implicit integrator in this context's solve_source: n one-wave workgroups for
- * lists of stiff cells longer than 8 n, else 2 n / 5 eight-wave workgroups (0: the default, five
+ * lists of stiff cells longer than 8 n, else 2 n / 5 eight-wave workgroups, or n / 4 four-wave ones
+ * for a mechanism beyond the eight-wave kernel's tables (0: the default, five
  * one-wave workgroups per compute unit; at most 2^24).  No counterpart in the reference: a tuning knob (a smaller grid leaves compute
  * units to concurrent work).  A cell's answer can differ in the last bits with the workgroup kind
  * that integrates it. */

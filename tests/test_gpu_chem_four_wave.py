@@ -1,0 +1,59 @@
+"""Short work lists of a mechanism that the eight-wave integrator's tables do not hold run four waves per
+cell.  Third-body efficiencies of 1 change no bit of a rate, so GRI-3.0 with three more of them in one row (ten;
+the tables hold eight) has to give the bits of GRI-3.0 itself, whose lists the eight-wave kernel sums in the
+order of the four-wave kernel's partial sums.  (One wave per cell sums the reactions in another order.)"""
+import os
+import shutil
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_chem import mixing_line_cells
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mechs(tmp_path_factory):
+    from fortrancfd_amd.lib import GRI30, Mechanism
+    d = tmp_path_factory.mktemp("mech") / "gri"
+    shutil.copytree(GRI30, d)
+    p = os.path.join(d, "chem.inp")
+    lines = open(p).read().splitlines()
+    at = next(i for i, l in enumerate(lines) if l.startswith("H2/ 2.40/ H2O/15.40/"))
+    lines.insert(at + 1, "O2/1.0/ N2/1.0/ OH/1.0/")
+    open(p, "w").write("\n".join(lines) + "\n")
+    return Mechanism(GRI30, text=True), Mechanism(str(d), text=True)
+
+
+@pytest.mark.parametrize("n", [1, 300])
+def test_batch(mechs, orc, n):
+    """One cell, and more cells than workgroups (256 four-wave ones)."""
+    plain, more = mechs
+    yT, rho, dt = mixing_line_cells(orc, n, 61)
+    yT[0, -1], dt[0] = 2400.0, 1e-6
+    print(f"{n} cells, GRI-3.0 with ten third bodies in a row", flush=True)
+    a, sa = plain.macks(dt, rho, yT)
+    b, sb = more.macks(dt, rho, yT)
+    assert (sa[:, 3] == 0).all() and (sa[:, 2] > 0).any()
+    np.testing.assert_array_equal(sa, sb)
+    np.testing.assert_array_equal(a, b)
+
+
+def test_domain(mechs):
+    """A coupled domain with the heat release of every step (the rates split into creation and
+    destruction) and step sizes kept from call to call."""
+    from fortrancfd_amd.lib import Solver
+    from tests.test_gpu_configs import ch4_air_cells
+    cells = ch4_air_cells(mechs[0].kk, 64, [(0, 12, 2100.0), (12, 4, 1600.0)])
+    out = []
+    for m in mechs:
+        print("coupled hot-spot domain, 64 cells", flush=True)
+        s = Solver(m, 2, 32, 25e-6, flag_acu=2, flag_weno=2, select_riemann=2, select_time=1, do_reaction=1)
+        s.set_step(strang=True, hrr_each_step=True)
+        s.init_cells(cells)
+        s.advance(0.5, 3)
+        out.append((*s.download(), *s.get_hrr()))
+    assert np.abs(out[0][2]).max() > 0
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
