@@ -59,11 +59,8 @@ __global__ void __launch_bounds__(64 * GW, WPE) k_flux(FluxArgs a) {
     const unsigned g0 = xcd_block() * 32u + unsigned(lane & 31);
     const bool live = g0 < total;
     const unsigned g = live ? g0 : total - 1u;            // lanes past the end shadow the last interface
-    // a launch covers blocks b0 .. b0 + nblk - 1 (the coarse blocks of a refined mesh reconstruct
-    // at first order in launches of their own, SRC/flux.f90:240)
     const unsigned bl = g / nif, j0 = g - bl * nif;
-    const unsigned gi = (unsigned(a.b0) + bl) * nif + j0; // interface index over all blocks
-    const unsigned c0 = (unsigned(a.b0) + bl) * unsigned(a.S) + unsigned(a.lv) + j0 - 1u;   // its left cell
+    const unsigned c0 = bl * unsigned(a.S) + unsigned(a.lv) + j0 - 1u;   // the interface's left cell
     CThermo *m = constant(a.thermo);
     const double *__restrict__ q = a.qf;
 
@@ -146,7 +143,7 @@ __global__ void __launch_bounds__(64 * GW, WPE) k_flux(FluxArgs a) {
         double *d = reinterpret_cast<double *>(reinterpret_cast<char *>(row) + at);
         *d = acc ? *d + val : val;
     };
-    const unsigned gb = gi * 8u;
+    const unsigned gb = g * 8u;
     if (w == 0) {
         Side me;
         me.rho = rho; me.u = u;
@@ -225,7 +222,7 @@ __global__ void __launch_bounds__(64 * GW, WPE) k_flux(FluxArgs a) {
             }
             if (a.godunov && s == 0) {                                // SRC/flux.f90:360-367
                 const double rt = sqrt(R.rho / L.rho);
-                double *G = a.godunov + gi;
+                double *G = a.godunov + g;
                 G[0] = sqrt(R.rho * L.rho);
                 G[PF] = (L.u + rt * R.u) / (1.0 + rt);
                 G[2 * PF] = (L.p + rt * R.p) / (1.0 + rt);
@@ -318,20 +315,6 @@ __device__ __forceinline__ void qc_to_qf_store(const DevThermo *__restrict__ m, 
     qf[2 * P + c] = temperature_con<NSP>(m, e, y);
 }
 
-// Source column of padded column (b, i): interior -> itself; wall ghost -> mirrored interior cell
-// with momentum negated (SRC/boundary.f90:152-199); block ghost -> the neighbour block's interior
-// cell (SRC/block.f90:490-497).
-__device__ __forceinline__ void ghost_source(const StageArgs &a, int b, int i, int &sb, int &si, double &sgn) {
-    sb = b; si = i; sgn = 1.0;
-    if (i < 0) {
-        if (b == 0) { si = -i - 1; sgn = -1.0; }
-        else { sb = b - 1; si = a.ncell + i; }
-    } else if (i >= a.ncell) {
-        if (b == a.nblk - 1) { si = 2 * a.ncell - 1 - i; sgn = -1.0; }
-        else { sb = b + 1; si = i - a.ncell; }
-    }
-}
-
 // Stage end: RK combine of the source cell, ghost fill, primitive recovery -- the interior update
 // of SRC/timeintegration.f90:150-175 (or :48-56 for Euler), then update_boundary /
 // interpolation_block / QcToqf on every column (:201-215).  mode 0: Q = Qin - dt/dx*dF;
@@ -347,16 +330,16 @@ __global__ void __launch_bounds__(64 * GW, WPE) k_stage_end(StageArgs a) {
     __shared__ CoopShared sh;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const unsigned ncol = unsigned(a.nblk) * unsigned(a.S);
-    const unsigned cq = xcd_block() * 64u + unsigned(lane);
-    const unsigned c = min(cq, ncol - 1u);                // lanes past the end shadow the last column
+    const unsigned cend = a.col0 + a.ncol;
+    const unsigned cq = a.col0 + xcd_block() * 64u + unsigned(lane);
+    const unsigned c = min(cq, cend - 1u);                // lanes past the end shadow the last column
     const int b = int(c / unsigned(a.S)), i = int(c - unsigned(b) * unsigned(a.S)) - a.lv;
     const bool ghost = (i < 0 || i >= a.ncell);
-    const bool live = cq < ncol && (ghost || !a.ghosts_only);
+    const bool live = cq < cend && (ghost || !a.ghosts_only);
     if (!__any(live)) return;                             // the same in the four waves
     int sb, si;
     double sgn;
-    ghost_source(a, b, i, sb, si, sgn);
+    ghost_source(a.left, a.right, a.ncell, b, i, sb, si, sgn);
     const unsigned sc = (unsigned(sb) * unsigned(a.S) + unsigned(a.lv + si)) * 8u;      // byte offsets
     const unsigned fj = (unsigned(sb) * unsigned(a.ncell + 1) + unsigned(si)) * 8u;
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
@@ -445,7 +428,7 @@ __global__ void __launch_bounds__(64) k_rk4_stage(StageArgs a) {
     }
     int sb, si;
     double sgn;
-    ghost_source(a, b, i, sb, si, sgn);
+    ghost_source(0, a.nblk - 1, a.ncell, b, i, sb, si, sgn);
     const long sc = long(sb) * a.S + a.lv + si;
     const long fj = long(sb) * (a.ncell + 1) + si;
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
@@ -538,19 +521,21 @@ __global__ void __launch_bounds__(64 * GW, 4) k_wave_speed(DtArgs a) {
     for (unsigned t0 = blockIdx.x * 64u; t0 < n; t0 += gridDim.x * 64u) {
         const unsigned t = min(t0 + unsigned(lane), n - 1u);      // a repeated cell changes no maximum
         const unsigned b = t / unsigned(a.ncell), i = t - b * unsigned(a.ncell);
-        const unsigned cb = (b * unsigned(a.S) + unsigned(a.lv) + i) * 8u;
+        const unsigned c = b * unsigned(a.S) + unsigned(a.lv) + i;
+        const unsigned cb = column_bytes(c, lane0(c));
+        const double *qf = a.qf + lane0(c);
         double y[M], x[M], s1[1];
         bool ok = true;
 #pragma unroll
         for (int j = 0; j < M; ++j) {
-            y[j] = at_byte(a.qf + long(3 + min(w * M + j, NSP - 1)) * a.P, cb);
+            y[j] = at_byte(qf + long(3 + min(w * M + j, NSP - 1)) * a.P, cb);
         }
 #pragma unroll
         for (int j = 0; j < M; ++j) {
             y[j] = w * M + j < NSP ? y[j] : 0.0;
             ok = ok && num_ok(y[j]);
         }
-        const double rho = at_byte(a.qf, cb), u = at_byte(a.qf + a.P, cb), T = at_byte(a.qf + 2 * a.P, cb);
+        const double rho = at_byte(qf, cb), u = at_byte(qf + a.P, cb), T = at_byte(qf + 2 * a.P, cb);
         const bool fast = __all(ok);
         over_wt_coop<NSP>(m, w, fast, y, x);
         chain_sum<1, M>(sh.c[0], w, lane, [&](int, int j) { return x[j]; }, s1);
@@ -692,7 +677,10 @@ __global__ void __launch_bounds__(64 * GW, 4) k_qf_to_qc_interior(const DevTherm
     const bool live = t0 < n;
     const unsigned t = live ? t0 : n - 1u;
     const unsigned b = t / unsigned(ncell);
-    const unsigned cb = (b * unsigned(S) + unsigned(lv) + (t - b * unsigned(ncell))) * 8u;
+    const unsigned c = b * unsigned(S) + unsigned(lv) + (t - b * unsigned(ncell));
+    const unsigned cb = column_bytes(c, lane0(c));
+    qf += lane0(c);
+    Qc += lane0(c);
     auto put = [cb, live](double *row, double v) {
         if (live) *reinterpret_cast<double *>(reinterpret_cast<char *>(row) + cb) = v;
     };
@@ -767,7 +755,7 @@ static int recon_kind(int flag_acu, int flag_weno) {
 }
 
 template <int NSP, bool SPH, int RK>
-static hipError_t launch_flux_rk(const FluxArgs &a, hipStream_t st) {
+static hipError_t launch_flux_slice(const FluxArgs &a, hipStream_t st) {
     const long n = long(a.nblk) * (a.ncell + 1);
     const dim3 grid(unsigned((n + 31) / 32)), blk(64 * GW);     // 32 interfaces, both sides, per workgroup
     switch (a.riemann) {
@@ -780,6 +768,30 @@ static hipError_t launch_flux_rk(const FluxArgs &a, hipStream_t st) {
             break;
     }
     return hipGetLastError();
+}
+
+// Launches of the blocks b0 .. b0 + nblk - 1 (the coarse blocks of a refined mesh reconstruct at first order in
+// launches of their own, SRC/flux.f90:240) over slices of them, and of a block alone where it is longer than a slice: the cells between its interfaces j and
+// j + n are a block of their own to the kernel.
+template <int NSP, bool SPH, int RK>
+static hipError_t launch_flux_rk(const FluxArgs &whole, hipStream_t st) {
+    return for_slices(whole.nblk, whole.S, SLICE, [&](int b, int n) {
+        FluxArgs a = whole;
+        const long blk = a.b0 + b;
+        a.qf += blk * a.S;
+        a.F += blk * (a.ncell + 1);
+        if (a.godunov) a.godunov += blk * (a.ncell + 1);
+        a.nblk = n;
+        if (a.S <= SLICE) return launch_flux_slice<NSP, SPH, RK>(a, st);
+        return for_slices(whole.ncell + 1, 1, SLICE, [&](int j, int m) {
+            FluxArgs p = a;
+            p.qf += j;
+            p.F += j;
+            if (p.godunov) p.godunov += j;
+            p.ncell = m - 1;
+            return launch_flux_slice<NSP, SPH, RK>(p, st);
+        });
+    });
 }
 
 template <int NSP, bool SPH>
@@ -817,12 +829,22 @@ hipError_t launch_flux(const FluxArgs &a, int nsp, int flag_acu, int flag_weno, 
 }
 
 template <int NSP, int MODE, bool SPH>
-static hipError_t launch_stage_end_mode(const StageArgs &a, hipStream_t st) {
-    const long n = long(a.nblk) * a.S;
-    const dim3 grid(unsigned((n + 63) / 64)), blk(64 * GW);     // 64 columns per workgroup
-    if (a.variant == 1) hipLaunchKernelGGL((k_stage_end<NSP, MODE, SPH, 4>), grid, blk, 0, st, a);
-    else hipLaunchKernelGGL((k_stage_end<NSP, MODE, SPH>), grid, blk, 0, st, a);
-    return hipGetLastError();
+static hipError_t launch_stage_end_mode(const StageArgs &whole, hipStream_t st) {
+    return for_slices(whole.nblk, whole.S, SLICE, [&](int b, int n) {
+        const StageSlice s = stage_slice(whole.nblk, whole.S, b, n);
+        StageArgs a = whole;
+        const long c = long(s.first) * a.S, f = long(s.first) * (a.ncell + 1);
+        if (a.Q0) a.Q0 += c;
+        a.Qin += c; a.Qout += c; a.qf += c; a.F += f;
+        if (a.god) a.god += f;
+        if (a.xm) a.xm += long(s.first) * a.ncell;
+        if (a.dxb) a.dxb += s.first;
+        a.col0 = s.col0; a.ncol = s.ncol; a.left = s.left; a.right = s.right;
+        const dim3 grid((s.ncol + 63u) / 64u), blk(64 * GW);    // 64 columns per workgroup
+        if (a.variant == 1) hipLaunchKernelGGL((k_stage_end<NSP, MODE, SPH, 4>), grid, blk, 0, st, a);
+        else hipLaunchKernelGGL((k_stage_end<NSP, MODE, SPH>), grid, blk, 0, st, a);
+        return hipGetLastError();
+    });
 }
 
 template <int NSP>

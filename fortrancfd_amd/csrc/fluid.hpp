@@ -15,7 +15,7 @@ struct FluxArgs {
     int muscl, riemann;
     int accumulate;       // 1: F += advection flux (transport flux already in F), 0: F = flux
     int spherical;        // 1: momentum flux rho u u without p (SRC/flux.f90:272-278)
-    int b0;               // first block of this launch (nblk blocks from there)
+    int b0;               // first block of the nblk blocks (launch_flux hands the kernel pointers from there on)
     int variant;          // register budget (WENO5 + HLLC only): 1 four waves per SIMD, else three
 };
 
@@ -35,6 +35,9 @@ struct StageArgs {
     int variant;           // register budget of k_stage_end: 1 four waves per SIMD, else three
     int nblk, ncell, lv, S;
     long P, PF;
+    // set by launch_stage_end: the launch's columns and the walls' blocks, from the slice's first block on
+    unsigned col0, ncol;
+    int left, right;
 };
 
 constexpr int DT_SLOTS = 32;                     // slots of the CFL maximum: (maximum, arrivals), 64 bytes apart

@@ -9,12 +9,16 @@
 // its block, hands the partial sum to wave 1 through LDS, and so on.
 #pragma once
 
+#include "columns.hpp"
 #include "fcfd_device.hpp"
 
 namespace fcfd {
 
 constexpr int GW = SPECIES_BLOCKS;                               // waves per workgroup
 template <int NSP> constexpr int group_m() { return (NSP + GW - 1) / GW; }   // species per wave
+
+// The value of lane 0: of indices that grow with the lane, a workgroup's smallest (column_bytes).
+__device__ __forceinline__ unsigned lane0(unsigned v) { return unsigned(__builtin_amdgcn_readfirstlane(int(v))); }
 
 // The thermo tables through the constant address space: reads at a wave-uniform index are scalar
 // loads wherever they stand (behind a store or a barrier the compiler would otherwise take them for

@@ -43,13 +43,16 @@ __global__ void __launch_bounds__(64 * GW, 3) k_tran_state(TranArgs a) {
     const bool live = t0 < n;
     const unsigned t = live ? t0 : n - 1u;
     const unsigned b = t / nc;
-    const unsigned cb = (b * unsigned(a.S) + unsigned(a.lv) - 1u + (t - b * nc)) * 8u;
+    const unsigned c = b * unsigned(a.S) + unsigned(a.lv) - 1u + (t - b * nc);
+    const unsigned cb = column_bytes(c, lane0(c));
+    const double *Qc = a.Qc + lane0(c);
+    double *props = a.props + lane0(t);
     double y[M], x[M], s1[1];
 #pragma unroll
-    for (int j = 0; j < M; ++j) y[j] = at_byte(a.Qc + long(3 + min(w * M + j, NSP - 1)) * a.P, cb);
-    const double rho = at_byte(a.Qc, cb);
-    const double u = at_byte(a.Qc + a.P, cb) / rho;
-    const double et = at_byte(a.Qc + 2 * a.P, cb) / rho;
+    for (int j = 0; j < M; ++j) y[j] = at_byte(Qc + long(3 + min(w * M + j, NSP - 1)) * a.P, cb);
+    const double rho = at_byte(Qc, cb);
+    const double u = at_byte(Qc + a.P, cb) / rho;
+    const double et = at_byte(Qc + 2 * a.P, cb) / rho;
     bool ok = den_ok(rho);
 #pragma unroll
     for (int j = 0; j < M; ++j) {
@@ -62,25 +65,25 @@ __global__ void __launch_bounds__(64 * GW, 3) k_tran_state(TranArgs a) {
     over_wt_coop<NSP>(m, w, fast, y, x);
     chain_sum<1, M>(sh.c[0], w, lane, [&](int, int j) { return x[j]; }, s1);
     ytx_coop<NSP>(m, w, fast, s1[0], y, x);
-    const unsigned pb = t * 8u;
+    const unsigned pb = column_bytes(t, lane0(t));
     auto put = [pb, live](double *row, double v) {
         if (live) *reinterpret_cast<double *>(reinterpret_cast<char *>(row) + pb) = v;
     };
 #pragma unroll
     for (int j = 0; j < M; ++j) {
         if (w * M + j >= NSP) break;
-        put(a.props + long(5 + w * M + j) * a.PP, y[j]);
-        put(a.props + long(5 + NSP + w * M + j) * a.PP, x[j]);
+        put(props + long(5 + w * M + j) * a.PP, y[j]);
+        put(props + long(5 + NSP + w * M + j) * a.PP, x[j]);
     }
     double wtm;
     const double ek = 0.5 * (u * u);
     const double T = temperature_coop<NSP>(m, sh, w, lane, et - ek, x, wtm);
     if (w == 0) {
-        put(a.props, rho);
-        put(a.props + a.PP, u);
-        put(a.props + 2 * a.PP, T);
-        put(a.props + 3 * a.PP, (rho * 1.e-3) * m->ru * T / wtm * 0.1);     // pressure (CKPX, SI)
-        put(a.props + 4 * a.PP, fm_log(T));
+        put(props, rho);
+        put(props + a.PP, u);
+        put(props + 2 * a.PP, T);
+        put(props + 3 * a.PP, (rho * 1.e-3) * m->ru * T / wtm * 0.1);     // pressure (CKPX, SI)
+        put(props + 4 * a.PP, fm_log(T));
     }
 }
 
@@ -231,10 +234,12 @@ __global__ void __launch_bounds__(64 * GW, 3) k_flux_tran(TranArgs a) {
     const bool live = t0 < n;
     const unsigned t = live ? t0 : n - 1u;
     const unsigned b = t / n1, j = t - b * n1;
-    const unsigned pb = (b * (n1 + 1u) + j) * 8u;      // cells ista-1+j and, 8 bytes on, ista+j
+    const unsigned c = b * (n1 + 1u) + j;              // cell ista-1+j; ista+j follows
+    const unsigned pb = column_bytes(c, lane0(c));
+    const double *props = a.props + lane0(c);
     const long PP = a.PP;
     auto pair = [&](int row, double &v0, double &v1) {
-        const double *q = a.props + long(row) * PP;
+        const double *q = props + long(row) * PP;
         v0 = at_byte(q, pb);
         v1 = at_byte(q + 1, pb);
     };
