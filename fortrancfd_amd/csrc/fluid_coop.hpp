@@ -50,9 +50,24 @@ __device__ __forceinline__ double quot(double n, double d, double r) {
     return __builtin_fma(__builtin_fma(-d, q, n), r, q);
 }
 
-// r refined to 1 / d from an estimate a few ulps off
+// r refined to 1 / d from an estimate at most 2^-51 off (relative).  Its error, half an ulp and 2^-102, leaves every
+// quotient right but for divisors whose mantissa is within 2^-49 of 2: with the mantissas of d and of a
+// quotient's middle as whole numbers the quotient is at least 1 / (2 d) ulps from the middle, and the closing step
+// moves it by half of r's relative error, at most d 2^-107 + 2^-103.
 __device__ __forceinline__ double refine(double d, double r) {
     return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+}
+
+// sqrt for x in the normal range: Goldschmidt's iteration on g -> sqrt(x), h -> 1 / (2 sqrt(x)) from the hardware's
+// estimate of 1 / sqrt(x), closed by two residual corrections (x - g g exact under the fused multiply-add).
+__device__ __forceinline__ double sqrt_core(double x) {
+    const double r = __builtin_amdgcn_rsq(x);
+    double g = x * r, h = 0.5 * r;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
 }
 
 // numerators: 0 or 2^-700 <= |v| <= 2^60; divisors: 2^-60 <= d <= 2^60.  With these every quotient,
@@ -223,11 +238,21 @@ __device__ __forceinline__ void ytx_coop(CThermo *m, int w, bool fast, double sw
     constexpr int M = group_m<NSP>();
     if (fast && __all(den_ok(sw))) {
         const double rs = recip(sw);
+        unsigned most = 0;        // the divisors' lower halves: refine() does not serve mantissas next to 2
 #pragma unroll
         for (int j = 0; j < M; ++j) {
             const int k = min(w * M + j, NSP - 1);
             const double d = sw * m->wt[k];
+            most = max(most, unsigned(__double2loint(d)));
             x[j] = quot(y[j], d, refine(d, rs * m->rwt[k]));
+        }
+        if (__any(most >= 0xfffffff0u)) {
+#pragma unroll
+            for (int j = 0; j < M; ++j) {
+                const double d = sw * m->wt[min(w * M + j, NSP - 1)];
+                x[j] = quot(y[j], d, recip(d));
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     } else {
 #pragma unroll

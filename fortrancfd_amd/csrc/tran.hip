@@ -87,18 +87,6 @@ __global__ void __launch_bounds__(64 * GW, 3) k_tran_state(TranArgs a) {
     }
 }
 
-// sqrt for x in the normal range, by the rounded sequence of the device library's sqrt without its
-// scaling and special values (the same bits).
-__device__ __forceinline__ double sqrt_core(double x) {
-    const double r = __builtin_amdgcn_rsq(x);
-    double g = x * r, h = 0.5 * r;
-    const double e = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, e, g);
-    h = __builtin_fma(h, e, h);
-    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
-}
-
 // Lane k < NSP is species k; it walks its row j = 0 .. NSP - 1 of the Wilke and binary-diffusion sums in
 // TRANLIB's order.  A row's table entries are read by neighbouring lanes and serve CPW cells; the
 // quotients and the square root go through reciprocals where a cell's values allow it (FAST), with
