@@ -822,9 +822,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
     }
 }
 
-// CKWYR and CKCDYR (cklib.f:9107-9204, 1422-1541) of n states through the integrator's own rate
+// CKWYR and CKCDYR (cklib.f:9107-9204, 1422-1541) of n states through this file's rate
 // code: rhs_begin (concentrations, S/R - H/RT, ctot), reaction / reaction_plain per row and
-// rhs_scatter into the production-rate sums, exactly as an integrator step evaluates them; the
+// rhs_scatter into the production-rate sums, as a step with one or four waves a cell evaluates them (the
+// eight-wave kernel and the screen have rate code of their own, tested through whole steps); the
 // rates of progress are also stored per reaction in the mechanism's order.  One state per wave.
 template <int NSP>
 __global__ void __launch_bounds__(64) k_rates(const DevThermo *__restrict__ th, const DevKin *__restrict__ K, int n,

@@ -182,7 +182,7 @@ int chem_coop_max(int n_workgroups, int nsp);
 hipError_t launch_zero_u32(unsigned *p, hipStream_t st, unsigned *q = nullptr);      // *p = 0, *q = 0
 // *out = f * *in on the device (one thread), e.g. the half step of Strang splitting.
 hipError_t launch_scale_scalar(const double *in, double *out, double f, hipStream_t st);
-// CKWYR / CKCDYR (cklib.f:9107-9204, 1422-1541) on n states with the integrator's own rate code:
+// CKWYR / CKCDYR (cklib.f:9107-9204, 1422-1541) on n states with the one-wave integrator's rate code:
 // rho [g/cm^3], T [K], Y [n][KK] in; wdot, cdot, ddot [n][KK] (mol/(cm^3 s)) and the rates of
 // progress qf, qr [n][II] (mechanism order) out.  One state per wave.
 hipError_t launch_rates(const DevThermo *th, const DevKin *K, int nsp, int n, const double *rho, const double *T,

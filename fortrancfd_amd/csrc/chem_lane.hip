@@ -252,7 +252,7 @@ __device__ __forceinline__ void rhs_lane(CThermo *th, CKin *K, LaneShared<NSP> &
     CSeries *ks = get_series();
     Temp tp = temperature(ks, T);
     // beyond any temperature of a state that can be accepted: NaN rates, the cell goes on to the integrator.
-    // (Arguments of exp_near stay below 2^30.)
+    // (Arguments of exp_near stay below 2^128 for activation temperatures below 2^121 K.)
     tp.logT = T >= 0x1p-7 && T <= 0x1p27 ? tp.logT : __builtin_nan("");
     const double lnT = tp.logT;
     const bool usual = K->usual != 0;

@@ -53,7 +53,8 @@ __device__ __forceinline__ double exp2term(CSeries *k, double x, double xl) {
     const double e = rh - (s - 1.0);
     return __builtin_amdgcn_ldexp(s + (e + (rl + (rh * rl + q))), int(kd));
 }
-// fm_exp for |x| < 2^30, NaN included: no clamp, one term
+// fm_exp for |x| < 2^128, NaN included: no clamp, one term.  (Far from 0 the reduction leaves more than ln2 / 2, but
+// the power of two decides: 0 or infinity.  Beyond 2^128 the series overflows.)
 __device__ __forceinline__ double exp_near(CSeries *k, double x) {
     const double kd = (x * k->inv_ln2 + k->shift) - k->shift;
     const double r0 = __builtin_fma(-kd, k->ln2_hi, x);
