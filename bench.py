@@ -146,21 +146,27 @@ def fluid_bytes(nequ, ntot, nblk, ncell):
 
 
 def measured_traffic(workload, kernel):
-    """HBM bytes per launch of `kernel` from the committed FETCH_SIZE / WRITE_SIZE summary of this
+    """HBM bytes per timed launch of `kernel` from the committed FETCH_SIZE / WRITE_SIZE summary of this
     workload (profiles/<workload>_hbm_traffic.json, two rocprofv3 --pmc runs scaled by a copy of
-    known size), or None."""
+    known size), or None: the mean over a kernel's instantiations by their dispatches (the stages of a
+    step), without those of a run's start, which are launched once."""
     path = os.path.join(REPO, "profiles", TRAFFIC_PROFILES.get(workload, ""))
     if not os.path.isfile(path):
         return None, None
     kernels = json.load(open(path))["kernels"]
     short = kernel.split(" ")[0]
-    # every kernel launched for the call (the integrator launches its one-wave and its eight-wave
-    # kernel each time; the one whose mode does not match the list returns at once)
-    hits = [rec["read_bytes"] + rec["write_bytes"] for name, rec in kernels.items()
-            if short + "<" in name or short + "_coop<" in name]
-    if not hits:
+
+    def mean(prefix):
+        recs = [r for name, r in kernels.items() if prefix in name and r["dispatches"] > 1]
+        n = sum(r["dispatches"] for r in recs)
+        return sum((r["read_bytes"] + r["write_bytes"]) * r["dispatches"] for r in recs) / n if n else None
+
+    # (the integrator launches its one-wave and its eight-wave kernel each time; the one whose mode does
+    # not match the list returns at once)
+    means = [m for m in (mean(short + "<"), mean(short + "_coop<")) if m is not None]
+    if not means:
         return None, None
-    return sum(hits), os.path.relpath(path, REPO)
+    return sum(means), os.path.relpath(path, REPO)
 
 
 TRAFFIC_PROFILES = {"inert1m": "fluid_inert1m_hbm_traffic.json",
