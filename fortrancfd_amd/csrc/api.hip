@@ -186,8 +186,8 @@ int ensure_dev_tables(const fcfd_mech *cm) {
 // next to the library's directory (FCFD_TUNE_FILE overrides), read once per process; entries for
 // other GPU architectures are ignored.  Keys: flux_variant, stage_variant (fluid.hpp),
 // chem_wg_per_cu (integrator workgroups per CU), chem_four_wave_factor (several waves per cell for
-// lists of at most factor x workgroups cells: eight, or four for a mechanism that the eight-wave integrator's
-// tables do not hold), chem_lu (kept for tables
+// lists of at most factor x workgroups cells: eight; four, for a sixth of that length, where the eight-wave
+// integrator's tables do not hold the mechanism), chem_lu (kept for tables
 // that hold it: the factorisations it chose between gave the same bits, and one is left).
 struct TuneTable {
     std::mutex mu;
@@ -484,7 +484,7 @@ hipError_t enqueue_source(fcfd_ctx *c, double dt, const double *dt_dev, bool wan
     const int chem_wg = c->chem_wg > 0 ? c->chem_wg : chem_workgroups(c->mech);
     a.route = c->d_accepted;
     const int n = c->nblk * c->ncell;
-    const int limit = chem_coop_max(chem_wg, c->kk);
+    const int limit = coop_limit(a, chem_wg, c->kk);
     a.f0 = n > limit ? c->d_f0 : nullptr;
     // explicit screen, one cell per lane: quiescent cells are final, the rest form the stiff list
     hipError_t e = timed(c, 6, [&]() {

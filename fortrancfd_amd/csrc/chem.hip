@@ -975,7 +975,7 @@ hipError_t launch_chem_full(ChemArgs a, int nsp, int n_workgroups, int *list, un
 // n_workgroups one-wave workgroups (five per CU by default) for long lists; two fifths as many eight-wave
 // workgroups -- two per CU, what its LDS and registers hold -- for lists of at most a.coop_max cells (the
 // tuned factor, default 8, times n_workgroups), or a quarter as many four-wave ones (122 kB of LDS, one per
-// CU) where the mechanism is beyond the eight-wave kernel's tables.  Up to coop_max the launch is set by its
+// CU) for a sixth of that length where the mechanism is beyond the eight-wave kernel's tables.  Up to coop_max the launch is set by its
 // slowest cells, which several waves take through a step several times as fast as one.  Both modes are
 // launched, and the one that does not match the list length on the device returns at once; where no list can
 // be long, only the one that can run (a launch that returns at once costs 4.5 us, 4 % of a small domain's
@@ -983,7 +983,7 @@ hipError_t launch_chem_full(ChemArgs a, int nsp, int n_workgroups, int *list, un
 hipError_t launch_chem(const ChemArgs &a0, int nsp, int n_workgroups, hipStream_t st) {
     hipError_t e;
     ChemArgs a = a0;
-    a.coop_max = chem_coop_max(n_workgroups, nsp);
+    a.coop_max = coop_limit(a, n_workgroups, nsp);
     if (a.order && a.list && a.list_n && a.stats && a.layout == 0) {
         hipLaunchKernelGGL(k_heavy_first, dim3(1), dim3(1024), 0, st, a.list, a.list_n, a.stats, a.order, a.counter);
         if ((e = hipGetLastError()) != hipSuccess) return e;

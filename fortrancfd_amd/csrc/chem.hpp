@@ -176,9 +176,15 @@ hipError_t launch_chem_screen(const ChemArgs &a, int nsp, hipStream_t st);
 // a.coop_max: accepted cells are final, the others go to a.stiff (a.stiff_n must be zero before
 // the launch) and *a.retry_done = 1; a shorter list is copied to a.stiff unchanged, *a.retry_done = 0.
 hipError_t launch_chem_retry(const ChemArgs &a, int nsp, hipStream_t st);
-// Longest list that gets a workgroup per cell: the tuned factor (default 8) times the workgroup count
+// Longest list that gets eight waves per cell: the tuned factor (default 8) times the workgroup count
 // (api.hip).
 int chem_coop_max(int n_workgroups, int nsp);
+// The same for these cells: a sixth of it, 1,706 cells by default, where a cell gets four waves.  Batches of GRI-3.0 with
+// ten third bodies, four waves and one: 1,536 cells 203 and 232 ms, 1,792: 231 and 235, 2,048: 272 and 240; 8,192:
+// 869 and 499.  (Eight waves are the faster at every length: 8,192 cells 292 ms and 499, 65,536: 2.08 s and 2.89.)
+inline int coop_limit(const ChemArgs &a, int n_workgroups, int nsp) {
+    return chem_coop_max(n_workgroups, nsp) / (a.coop ? 1 : 6);
+}
 hipError_t launch_zero_u32(unsigned *p, hipStream_t st, unsigned *q = nullptr);      // *p = 0, *q = 0
 // *out = f * *in on the device (one thread), e.g. the half step of Strang splitting.
 hipError_t launch_scale_scalar(const double *in, double *out, double f, hipStream_t st);

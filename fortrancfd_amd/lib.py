@@ -309,8 +309,8 @@ class Solver:
 
     def set_chem_workgroups(self, n):
         """Grid of the implicit integrator (0: default): n one-wave workgroups for lists longer
-        than 8 n cells, else 2 n / 5 eight-wave workgroups (n / 4 four-wave ones for a mechanism
-        beyond the eight-wave kernel's tables)."""
+        than 8 n cells, else 2 n / 5 eight-wave workgroups; for a mechanism beyond the eight-wave
+        kernel's tables n / 4 four-wave ones up to 8 n / 6 cells."""
         _check(lib().fcfd_set_chem_workgroups(self.handle, C.c_int(n)))
 
     def source_accepted(self):

@@ -227,9 +227,11 @@ int fcfd_set_timing(fcfd_ctx *c, int enable);
  * per SIMD with 1, three with 0 or 2), "stage_variant" (stage update: four waves per SIMD with 1,
  * three with 0, 2 or 3), "chem_wg_per_cu" (implicit-integrator workgroups per CU, default 5),
  * "chem_four_wave_factor" (several waves per cell for lists of at most factor x workgroups cells, default
- * 8: eight waves, or four for a mechanism that the eight-wave kernel's tables do not hold), "chem_lu" (accepted and without effect: it chose between
- * factorisations of the same bits, of which one is left; default 2).  fcfd_set_launch overrides one entry for the mechanisms of nsp species (every context
- * re-captures its step graph); fcfd_load_tuning reloads the table (NULL: the default file). */
+ * 8: eight waves; four, and a sixth of that length, for a mechanism that the eight-wave kernel's tables do
+ * not hold -- more than 384 reactions, 8 third-body efficiencies in a reaction or 32 fall-off reactions, a
+ * coefficient above 3), "chem_lu" (accepted and without effect: it chose between factorisations of the same
+ * bits, of which one is left; default 2).  fcfd_set_launch overrides one entry for the mechanisms of nsp
+ * species (every context re-captures its step graph); fcfd_load_tuning reloads the table (NULL: the default file). */
 int fcfd_set_launch(const char *key, int nsp, int value);
 int fcfd_get_launch(const char *key, int nsp, int *value);
 int fcfd_load_tuning(const char *path);
@@ -349,8 +351,8 @@ int fcfd_set_surrogate(fcfd_ctx *c, fcfd_surrogate *s);
  * with 0. */
 int fcfd_source_accepted(fcfd_ctx *c, int *per_cell, int *n_fallback);
 /* Grid of the FP64 implicit integrator in this context's solve_source: n one-wave workgroups for
- * lists of stiff cells longer than 8 n, else 2 n / 5 eight-wave workgroups, or n / 4 four-wave ones
- * for a mechanism beyond the eight-wave kernel's tables (0: the default, five
+ * lists of stiff cells longer than 8 n, else 2 n / 5 eight-wave workgroups; for a mechanism beyond the
+ * eight-wave kernel's tables n / 4 four-wave ones up to 8 n / 6 (0: the default, five
  * one-wave workgroups per compute unit; at most 2^24).  No counterpart in the reference: a tuning knob (a smaller grid leaves compute
  * units to concurrent work).  A cell's answer can differ in the last bits with the workgroup kind
  * that integrates it. */
@@ -358,7 +360,7 @@ int fcfd_set_chem_workgroups(fcfd_ctx *c, int n);
 
 /* Plain BF16 GEMM C (FP32) = A B on device arrays with element (m, k) of A at A[m*sam + k*sak]
  * and (k, n) of B at B[k*sbk + n*sbn]; M, N multiples of 64, K / ksplit a multiple of 16;
- * split s of K writes C + s*M*ldc.  The kernel the surrogate's layers run on. */
+ * split s of K writes C + s*M*ldc.  (The surrogate's layers run in a kernel of their own.) */
 int fcfd_bf16_gemm(int M, int N, int K, const void *A, long sam, long sak, const void *B,
                    long sbk, long sbn, float *C, long ldc, int ksplit, void *stream);
 

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from tests.test_gpu_chem import mixing_line_cells
+from tests.test_gpu_launch_variants import restore_table, set_launch  # noqa: F401 (fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -36,6 +37,21 @@ def test_batch(mechs, orc, n):
     a, sa = plain.macks(dt, rho, yT)
     b, sb = more.macks(dt, rho, yT)
     assert (sa[:, 3] == 0).all() and (sa[:, 2] > 0).any()
+    np.testing.assert_array_equal(sa, sb)
+    np.testing.assert_array_equal(a, b)
+
+
+def test_longer_list(mechs, orc):
+    """Past the length up to which four waves are the faster: one wave per cell."""
+    plain, more = mechs
+    yT, rho, dt = mixing_line_cells(orc, 2600, 62)
+    yT[:, -1] = np.maximum(yT[:, -1], 1800.0)               # (most cells reach the list)
+    dt[:] = 1e-7
+    print("2,600 cells, GRI-3.0 with ten third bodies in a row", flush=True)
+    b, sb = more.macks(dt, rho, yT)
+    set_launch("chem_four_wave_factor", 0)
+    a, sa = plain.macks(dt, rho, yT)
+    assert (sa[:, 2] > 0).sum() > 8 * 1280 // 6
     np.testing.assert_array_equal(sa, sb)
     np.testing.assert_array_equal(a, b)
 
