@@ -22,7 +22,8 @@
 // about 38k; some seven Newton iterations an attempt.  Four waves that each evaluated blocks of rows,
 // scattered into their own partial sums and Jacobian (155 kB of LDS, one workgroup per CU) and ran the
 // integrator redundantly took 18.8k, 6.3k, 67k and 58k.  256 cells of the chemistry batch: 111 -> 62
-// ms; 3,000 cells, which two workgroups per CU serve: 375 -> 137 ms; 200 H2/O2 cells: 24.5 -> 12.4 ms.
+// ms; 3,000 cells, which two workgroups per CU serve: 375 -> 137 ms; 200 H2/O2 cells: 24.5 -> 12.4 ms.  (That
+// kernel, k_chem<NSP, 4>, still takes the mechanisms that the tables here do not hold.)
 #include <algorithm>
 
 #include "chem_wave.hpp"

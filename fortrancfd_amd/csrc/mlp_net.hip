@@ -84,8 +84,10 @@ __device__ __forceinline__ void layer(Stream<D> &s, const v4s (&act)[FB][RT], v4
 // A workgroup of four waves: 16 RT rows a wave (RT = 1: 64 rows, 2: 128), or 16 rows for FS waves that share
 // the features of each layer and pass their activations to each other through LDS (FS = 2: 32 rows, 4: 16).
 // Bound: the activation function -- erff takes some 45 vector operations, 1,024 of them a row -- and the
-// half-rate MFMA of this depth, which keeps the sums' order: for 65,536 rows about 65 and 29 us.  There
-// 110 us a pass; five GEMMs of 64 x 64 tiles, loading two bytes a lane and passing every layer through
+// half-rate MFMA of this depth, which keeps the sums' order: for 65,536 rows about 65 and 29 us.  With 128 rows
+// the accumulators and activations do not all fit 256 registers: inference, training's forward and backward keep
+// 132, 172 and 156 bytes a lane in scratch, traffic that those figures leave out.  (64 rows and fewer: 136 to
+// 186 registers, no scratch.)  65,536 rows: 110 us a pass; five GEMMs of 64 x 64 tiles, loading two bytes a lane and passing every layer through
 // memory, took 5 x 72 us.
 template <int MODE, int RT, int FS>
 __global__ void __launch_bounds__(256, 2) k_mlp(NetArgs a) {
@@ -197,8 +199,11 @@ __global__ void __launch_bounds__(256, 2) k_mlp(NetArgs a) {
 }
 
 // As many rows a workgroup as still give each of 256 CUs one: 16 or 32 (features split), 64, else 128, which
-// stream the weights least often (8,192 rows, training's forward: 64 rows a workgroup 61 us, 32 rows 41;
-// 65,536 rows, inference: 64 rows 116 us, 128 rows 110).
+// stream the weights least often.  Both sides, by calls: 8,192 rows, training's forward: 64 rows a workgroup 61 us,
+// 32 rows 41; 65,536 rows, inference: 64 rows 128 us, 128 rows 125.  The line between 64 and 128 serves large
+// inference only: just above it two rounds of 64 rows are the faster (32,768 rows, inference: 73 us, 128 rows
+// 103), and training's passes, which spill more, are so throughout (four steps of 32,768 rows 1.37 ms, 128 rows
+// 1.91; of 65,536: 2.46 and 2.95).
 template <int MODE>
 static hipError_t launch_net(const NetArgs &a, hipStream_t st) {
     if (a.rows <= 0 || a.rows % 64) return hipErrorInvalidValue;

@@ -94,8 +94,9 @@ __global__ void __launch_bounds__(64 * GW, 3) k_tran_state(TranArgs a) {
 // cell's wave repeated the temperature iteration and gathered its D fit per lane, with two square
 // roots and three divisions per pair: 786 us for 16,384 cells, 90 us for 510 (now k_tran_state and
 // this kernel, 195 and 47 us).  Forming D_jk once for
-// both rows (rotating it between the lanes, the sums in offset order) is 1.5 times faster again, but
-// other sums round differently, and a flame's heat release feels it.
+// both rows and rotating it between the lanes, the sums in offset order, is 1.5 times faster again, but
+// those sums round differently, and a flame's heat release feels it.  (Kept in LDS, D_jk could be summed in
+// TRANLIB's order: not tried.)
 template <int NSP, int CPW>
 struct PairLds {
     double2 xv[4 * CPW][64];                            // X_j, 1 / vis_j

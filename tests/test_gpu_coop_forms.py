@@ -16,9 +16,9 @@ from tests.test_gpu_mech2 import states
 pytestmark = pytest.mark.gpu
 
 
-def edit_link_file(src, dst, falloff=None, reaction=None):
+def edit_link_file(src, dst, falloff=None, reaction=None, third=None):
     """A copy of a mechanism's folder with rows of its link file changed: falloff(f, form, species, par) and
-    reaction(i, par) return the new values."""
+    reaction(i, par) return the new values, third(t, bodies) the row's list of (species, efficiency)."""
     shutil.copytree(src, dst)
     path = os.path.join(dst, "chem.bin")
     data, at, records = bytearray(open(path, "rb").read()), 0, []
@@ -27,7 +27,7 @@ def edit_link_file(src, dst, falloff=None, reaction=None):
         records.append(at + 4)
         at += n + 8
     size = struct.unpack_from("<29i", data, records[1])
-    ii, npar, nfar, nfal = size[5], size[10], size[12], size[14]
+    ii, mxtb, npar, nfar, nfal, ntb = size[5], size[7], size[10], size[12], size[14], size[15]
     for i in range(ii if reaction else 0):
         p = records[4] + i * (8 + 8 * npar + 48) + 8
         struct.pack_into(f"<{npar}d", data, p, *reaction(i, list(struct.unpack_from(f"<{npar}d", data, p))))
@@ -37,8 +37,38 @@ def edit_link_file(src, dst, falloff=None, reaction=None):
         par = list(struct.unpack_from(f"<{nfar}d", data, p + 12))
         form, sp, par = falloff(f, form, sp, par)
         struct.pack_into(f"<2i{nfar}d", data, p + 4, form, sp, *par)
+    for t in range(ntb if third else 0):
+        p = records[6] + t * (8 + 12 * mxtb) + 4
+        bodies = [struct.unpack_from("<id", data, p + 4 + 12 * l) for l in range(struct.unpack_from("<i", data, p)[0])]
+        bodies = third(t, bodies)
+        struct.pack_into("<i", data, p, len(bodies))
+        for l, (k, a) in enumerate(bodies):
+            struct.pack_into("<id", data, p + 4 + 12 * l, k, a)
     open(path, "wb").write(data)
     return str(dst)
+
+
+def second_passes(M):
+    """Whether the eight-wave factorisation of M takes a panel again: (a pivot outside 2^-100 .. 2^102 or a multiplier
+    below 2^-790 but 0, two open rows of the pivot's upper 32 bits)."""
+    M, n = M.copy(), len(M)
+    rows, scale, ties = list(range(n)), False, False
+    for k in range(n):
+        p = max(rows, key=lambda r: abs(M[r, k]))
+        high = np.abs(M[rows, k]).view(np.int64) >> 32
+        ties |= bool((high == high.max()).sum() > 1)
+        rows.remove(p)
+        scale |= not 2.0 ** -100 <= abs(M[p, k]) < 2.0 ** 102
+        for r in rows:
+            f = M[r, k] / M[p, k]
+            scale |= 0.0 < abs(f) < 2.0 ** -790
+            M[r, k:] -= f * M[p, k:]
+    return scale, ties
+
+
+def newton_matrix(o, dt, rho, yT):
+    """Of the first step over dt."""
+    return np.eye(o.kk + 1) - 0.4358665 * dt * o.chem_jac(rho * 1e-3, yT)
 
 
 def forms(h2o):
@@ -114,22 +144,33 @@ def test_domain(tmp_path, factor):
     compare_fields(s, d, dts_o, dts_o, o)
 
 
-def usual_panels(M):
-    """Whether the eight-wave factorisation of M keeps its first pass: pivots in 2^-100 .. 2^102, no multiplier
-    below 2^-790 but 0 (ties aside)."""
-    M, n = M.copy(), len(M)
-    rows = list(range(n))
-    for k in range(n):
-        p = max(rows, key=lambda r: abs(M[r, k]))
-        rows.remove(p)
-        if not 2.0 ** -100 <= abs(M[p, k]) < 2.0 ** 102:
-            return False
-        for r in rows:
-            f = M[r, k] / M[p, k]
-            if 0.0 < abs(f) < 2.0 ** -790:
-                return False
-            M[r, k:] -= f * M[p, k:]
-    return True
+def test_ties(tmp_path, orc):
+    """HCNO + H = H + HNCO so fast that 1 - hg J loses its 1: two species of one mass, two equal pivot
+    candidates.  The four-wave kernel's sums have the eight-wave kernel's order; it runs for the same mechanism with
+    ten third bodies in a row, three of them of efficiency 1."""
+    from fortrancfd_amd.lib import GRI30, Mechanism
+    from oracle.pyoracle import Oracle
+    m = Mechanism(GRI30)
+    par, nu, nk, ns, nr = orc.arrhenius()
+    a, b, h = (m.names.index(s) + 1 for s in ("HCNO", "HNCO", "H"))
+    at = [i for i in range(m.ii) if a in nk[i] and b in nk[i] and h in nk[i]]
+    assert len(at) == 1
+    fast = lambda i, p: [1e36, 0.0, 0.0] if i == at[0] else p
+    ones = [m.names.index(s) + 1 for s in ("O2", "N2", "OH")]
+    more = lambda t, rows: rows + [(k, 1.0) for k in ones] if t == 0 else rows
+    dirs = [edit_link_file(GRI30, tmp_path / "eight", reaction=fast), edit_link_file(GRI30, tmp_path / "four", reaction=fast, third=more)]
+    o = Oracle(dirs[0])
+    yT, rho, dt = mixing_line_cells(orc, 32, 94)
+    yT[:, h - 1] += 1e-4
+    dt = np.maximum(dt, 1e-7)
+    assert sum(second_passes(newton_matrix(o, dt[c], rho[c], yT[c])) == (False, True) for c in range(32)) > 16
+    out = []
+    for d in dirs:
+        print(f"32 cells, {os.path.basename(d)} waves", flush=True)
+        out.append(Mechanism(d).macks(dt, rho, yT))
+    assert (out[0][1][:, 2] > 0).sum() > 16
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    np.testing.assert_array_equal(out[0][0], out[1][0])
 
 
 @pytest.mark.parametrize("kind", ["trace", "stiff", "nan"])
@@ -149,7 +190,7 @@ def test_second_factorisation(tmp_path, kind):
             Y[:, m.names.index(sp)] = 10.0 ** -np.linspace(200.0, 270.0, 40)
     yT = np.column_stack([Y, T])
     if kind != "nan":
-        odd = [not usual_panels(np.eye(m.kk + 1) - 0.4358665 * dt[c] * o.chem_jac(rho[c] * 1e-3, yT[c])) for c in range(40)]
+        odd = [second_passes(newton_matrix(o, dt[c], rho[c], yT[c]))[0] for c in range(40)]
         assert sum(odd) > 10
     else:
         yT, rho, dt = yT[:2], rho[:2], dt[:2]
